@@ -5,6 +5,7 @@
 #include "kind_launch.h"
 #define INGOT_KIND_UNIT  // leave out the format-independent kernels
 #include "moe_kernels.cuh"
+#include "gemm_small.cuh"
 
 namespace ingot {
 
@@ -183,12 +184,41 @@ bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, 
 #undef F16L
 }
 
+template <int KIND, bool GATEUP>
+void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a) {
+#define SML_(AO, TLV)                                                                                            \
+    hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
+                       a.e_shared, a.stride0, a.stride1, a.rows_per_expert, a.kdim, a.ah, a.al, a.gs, a.pairs,   \
+                       a.K, a.tiles, a.ldo, a.limit, a.out, a.out_h, a.out_l, a.out_gs, a.nblk, a.a_rows,        \
+                       a.xstat, a.rowmax, a.flags, a.slot_of)
+#define SML(AO)                 \
+    do {                        \
+        if (tl) SML_(AO, true); \
+        else SML_(AO, false);   \
+        return;                 \
+    } while (0)
+    if constexpr (GATEUP) {
+        switch (aord) {
+            case A_IQ4NL: SML(A_IQ4NL);
+            case A_IQ3XXS: SML(A_IQ3XXS);
+            case A_Q6K: SML(A_Q6K);
+            default: SML(A_NATURAL);
+        }
+    } else {
+        SML(A_NATURAL);
+    }
+#undef SML
+#undef SML_
+}
+
 }  // namespace ingot
 
 #define INGOT_INSTANTIATE_F16(K)                                                                          \
     namespace ingot {                                                                                     \
     template bool launch_gemm_f16_k<K, true>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&);  \
     template bool launch_gemm_f16_k<K, false>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&); \
+    template void launch_gemm_small_k<K, true>(hipStream_t, int, bool, dim3, const GemmF16Args&);               \
+    template void launch_gemm_small_k<K, false>(hipStream_t, int, bool, dim3, const GemmF16Args&);              \
     }
 
 #define INGOT_INSTANTIATE_KIND(K)                                                                                \

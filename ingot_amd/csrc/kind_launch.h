@@ -26,6 +26,7 @@
 
 namespace ingot {
 
+constexpr uint32_t TMS = 16;   // pairs per tile of the small-tile GEMM
 constexpr int GEMV_RPW = 4;  // rows per wave of the separate gate/up GEMV (1 when that leaves CUs idle)
 constexpr int DEC_RPW = 1;   // down rows per wave of the decode down kernel
 
@@ -136,10 +137,15 @@ struct GemmF16Args {
 // always), else 64; false if no instantiation covers the arguments.
 template <int KIND, bool GATEUP>
 bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, const GemmF16Args& a);
+// k_gemm_small<KIND, GATEUP, aord, tl>: the same over tiles of at most TMS pairs.
+template <int KIND, bool GATEUP>
+void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a);
 
 #define INGOT_DECLARE_F16(K)                                                                                \
     extern template bool launch_gemm_f16_k<K, true>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&); \
-    extern template bool launch_gemm_f16_k<K, false>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&);
+    extern template bool launch_gemm_f16_k<K, false>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&); \
+    extern template void launch_gemm_small_k<K, true>(hipStream_t, int, bool, dim3, const GemmF16Args&);           \
+    extern template void launch_gemm_small_k<K, false>(hipStream_t, int, bool, dim3, const GemmF16Args&);
 
 #define INGOT_DECLARE_KIND(K)                                                                               \
     extern template bool launch_gemv_gate_up_k<K>(hipStream_t, uint32_t, uint32_t, dim3, const GateUpArgs&); \

@@ -392,6 +392,17 @@ bool launch_gemm_f16(hipStream_t s, uint32_t kind, int aord, bool tt128, bool tl
     }
 }
 
+// The same over tiles of at most TMS pairs (k_gemm_small).
+template <bool GATEUP, typename... Args>
+void launch_gemm_small(hipStream_t s, uint32_t kind, int aord, bool tl, dim3 grid, Args... args) {
+    const GemmF16Args a{args...};
+    switch (kind) {
+#define K_(KV) case KV: launch_gemm_small_k<KV, GATEUP>(s, aord, tl, grid, a); return;
+        INGOT_F16_KINDS(K_)
+#undef K_
+    }
+}
+
 }  // namespace
 
 // Rows per wave: 3 when that spreads the blocks more evenly over the 256 CUs
@@ -675,6 +686,15 @@ static uint64_t carve(const ingot_layer* L, uint32_t T, void* base, Ws* out) {
 // experts, top-10) at 2 / 4 / 6 tokens 30.3 / 47.6 / 65.0 against 112.5 /
 // 124.9 / 128.7.
 static const uint32_t GEMV_MAX_PAIRS = 64;
+
+// Batches of up to this many pairs per expert on average run k_gemm_small,
+// larger ones k_gemm_f16. Gate/up + down us, k_gemm_f16 against k_gemm_small:
+// 128 experts top-8 at 4 / 8 / 12 / 16 pairs per expert, Q4_K 104 / 108 / 110 /
+// 119 against 80 / 86 / 95 / 118, the Zipf-biased router 60 / 70 / - / 89 against
+// 41 / 58 / 73 / 90; IQ3_XXS / IQ4_NL at H = 4096, 4 / 8 / 16: 266 / 314 / 386
+// against 227 / 302 / 459; 512 IQ2_XS experts top-10 at 1.2 / 5 / 10: 269 / 328 /
+// 342 against 220 / 262 / 296.
+static const uint32_t SMALL_PAIRS_PER_EXPERT = 12;
 
 // Whether a forward of T tokens takes the decode kernels (else routing,
 // dispatch and the grouped GEMMs). A cached layer reads the routing back to
@@ -1550,10 +1570,15 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         // / 131. (A Q6_K projection runs its 128-token kernel on either.)
         const bool tt128 = f16 && T > TM && (uint64_t)T * K >= 32ull * E && f16_tt128_kind(gate.kind) &&
                            f16_tt128_kind(down.kind);
-        const uint32_t tm = tt128 ? 2u * TM : TM;
         // The f16 GEMMs read the tiled copies where every matrix of the launch has one.
         const bool tlg = f16gu && gate.t && up.t && (!merge || (sgate.t && sup.t));
         const bool tld = f16 && down.t && (!merge || sdown.t);
+        // The small-tile GEMM up to SMALL_PAIRS_PER_EXPERT pairs per expert on average;
+        // its tile list lies in w.act, which only an fp32 down GEMM uses.
+        const uint32_t pcap = (P + TMS - 1) / TMS + E + (merge ? (T + TMS - 1) / TMS : 0u);
+        const bool small = f16 && P <= SMALL_PAIRS_PER_EXPERT * E && 16ull * pcap <= 4ull * P * F;
+        uint32_t* const ptiles = small ? reinterpret_cast<uint32_t*>(w.act) : nullptr;
+        const uint32_t tm = tt128 ? 2u * TM : TM;
         const uint8_t *g16 = tlg ? gate.t : gate.d, *u16 = tlg ? up.t : up.d, *d16 = tld ? down.t : down.d;
         const uint8_t *sg16 = tlg ? sgate.t : sgate.d, *su16 = tlg ? sup.t : sup.d, *sd16 = tld ? sdown.t : sdown.d;
         const uint32_t S = merge ? T : 0u, capf = cap + (merge ? scap : 0u), e_sh = merge ? E : 0xffffffffu;
@@ -1575,7 +1600,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             const uint32_t nsplit = (uint32_t)((n / 4 + 1023) / 1024);
             hipLaunchKernelGGL(k_dispatch, dim3(1 + nsplit), dim3(1024), 0, ss, ids, P, E, tm, capf, counts, first, tiles,
                                pairs, inverse, S, K, xin, n, xh, xl, xs, (uint32_t)xord, (const float*)xstat, H, rmx,
-                               nrow);
+                               nrow, ptiles, pcap);
             if (hs && !merge)
                 hipLaunchKernelGGL(k_dense_tiles, dim3((scap + 63) / 64), dim3(64), 0, ss, T, scap, stiles);
         };
@@ -1583,7 +1608,14 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         ingot_layer* const LL = L;
         L->stage[ST_GATEUP] = [=](hipStream_t ss) {
             const uint32_t* so = LL->pass.slot_of;
-            if (f16gu) {
+            if (small) {
+                launch_gemm_small<true>(ss, gate.kind, aord, tlg, dim3(8 * (F / 64) * ((pcap + 7) / 8)), g16, u16,
+                                        merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride, F,
+                                        H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
+                                        (const uint32_t*)pairs, K, (const uint32_t*)ptiles, F, limit, (float*)nullptr,
+                                        acth, actl, mins ? acts : nullptr, F / 64, T, (const float*)xstat, rmx, flags,
+                                        so);
+            } else if (f16gu) {
                 launch_gemm_f16<true>(ss, gate.kind, aord, tt128, tlg, dim3(8 * (F / 64) * ((capf + 7) / 8)), g16, u16,
                                       merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride,
                                       F, H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
@@ -1601,7 +1633,14 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         L->stage_name[ST_GATEUP] = f16gu ? "k_gemm_f16<gate_up>" : "k_gemm<gate_up>";
         L->stage[ST_DOWN] = [=](hipStream_t ss) {
             const uint32_t* so = LL->pass.slot_of;
-            if (f16)
+            if (small)
+                launch_gemm_small<false>(ss, down.kind, A_NATURAL, tld, dim3(8 * (H / 128) * ((pcap + 7) / 8)), d16,
+                                         (const uint8_t*)nullptr, merge ? sd16 : nullptr, (const uint8_t*)nullptr, e_sh,
+                                         down.stride, 0ull, H, F, (const _Float16*)acth, (const _Float16*)actl,
+                                         (const float*)acts, (const uint32_t*)nullptr, K, (const uint32_t*)ptiles, H, 0.f,
+                                         Y, (_Float16*)nullptr, (_Float16*)nullptr, (float*)nullptr, H / 128,
+                                         (uint32_t)(P + S), (const float*)xstat, rmx, flags, so);
+            else if (f16)
                 launch_gemm_f16<false>(ss, down.kind, A_NATURAL, tt128, tld, dim3(8 * (H / 128) * ((capf + 7) / 8)), d16,
                                        (const uint8_t*)nullptr, merge ? sd16 : nullptr, (const uint8_t*)nullptr, e_sh,
                                        down.stride, 0ull, H, F, (const _Float16*)acth, (const _Float16*)actl,

@@ -1602,7 +1602,8 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
                                                    _Float16* __restrict__ xh, _Float16* __restrict__ xl,
                                                    float* __restrict__ xs, uint32_t xorder,
                                                    const float* __restrict__ xstat, uint32_t H,
-                                                   uint32_t* __restrict__ rowmax, uint32_t nrow) {
+                                                   uint32_t* __restrict__ rowmax, uint32_t nrow,
+                                                   uint32_t* __restrict__ stiles, uint32_t scap) {
     if (blockIdx.x > 0) {
         split_f16_part(x, xn, xh, xl, xs, xorder, (uint64_t)(blockIdx.x - 1u) * blockDim.x + threadIdx.x, xstat, H);
         return;
@@ -1613,6 +1614,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
     __shared__ uint32_t wsum[32];
     __shared__ uint32_t tot[3];
     __shared__ uint32_t rbin[1024];  // partial tiles per remainder, then their start positions
+    __shared__ uint32_t sbin[TMS];   // the same positions in stiles
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
 #pragma unroll
     for (int w = 0; w < 16; ++w) hist[w][tid] = 0;
@@ -1643,9 +1645,13 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
         }
     }
     const uint32_t nfull = n / TM, rem = n - nfull * TM;
+    // stiles != NULL: also the tile list of the small-tile GEMM (tiles of TMS
+    // pairs, the same order); its counts ride in the upper halves of the scans.
+    const uint32_t sfull = n / TMS, srem = n - sfull * TMS, half = stiles ? 0xffffu : 0xffffffffu;
     const uint32_t f = block_exclusive_scan_1024(n, wsum, &tot[0]);
     __syncthreads();
-    const uint32_t t0 = block_exclusive_scan_1024(nfull, wsum, &tot[1]);  // full tiles
+    const uint32_t t0s = block_exclusive_scan_1024(nfull + (stiles ? sfull << 16 : 0u), wsum, &tot[1]);  // full tiles
+    const uint32_t t0 = t0s & half;
     if (tid < E) {
         counts[tid] = n;
         first[tid] = f;
@@ -1653,20 +1659,36 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
         for (int w = 0; w < 16; ++w) hist[w][tid] += f;
     }
     if (rem) atomicAdd(&rbin[rem], 1u);
+    if (stiles && srem) atomicAdd(&rbin[srem], 1u << 16);
     __syncthreads();
     // Start of each remainder's run among the partial tiles (larger remainders
     // first): exclusive scan over remainders TM-1 .. 1.
     const uint32_t rr = tid < TM ? TM - 1u - tid : 0u;
-    const uint32_t c = (tid < TM && rr > 0) ? rbin[rr] : 0u;
+    uint32_t c = (tid < TM && rr > 0) ? rbin[rr] & half : 0u;
+    if (stiles && tid < TMS - 1u) c += rbin[TMS - 1u - tid] & 0xffff0000u;
     const uint32_t before = block_exclusive_scan_1024(c, wsum, &tot[2]);
-    const uint32_t nt_all = tot[2];
+    const uint32_t nt_all = tot[2] & half, nfull_all = tot[1] & half;
     __syncthreads();
     // The shared expert's S rows (S = 0: none) come first, as expert E over
     // positions P..P+S-1, whose pairs entry t K names token t.
     const uint32_t nsh = (S + TM - 1u) / TM;
-    if (tid < TM && rr > 0) rbin[rr] = nsh + tot[1] + before;
+    const uint32_t ssh = (S + TMS - 1u) / TMS, sfull_all = tot[1] >> 16;
+    if (tid < TM && rr > 0) rbin[rr] = nsh + nfull_all + (before & half);
+    if (stiles && tid < TMS - 1u) sbin[TMS - 1u - tid] = ssh + sfull_all + (before >> 16);
     __syncthreads();
-    const uint32_t ntiles = min(nsh + tot[1] + nt_all, cap);
+    if (stiles) {
+        const uint32_t nst = min(ssh + sfull_all + (tot[2] >> 16), scap);
+        auto put = [&](uint32_t t, uint32_t e, uint32_t q, uint32_t m) {
+            if (t < scap) *reinterpret_cast<uint4*>(stiles + 4u * t) = make_uint4(e, q, m, nst);
+        };
+        for (uint32_t j = tid; j < ssh; j += 1024u) put(j, E, P + j * TMS, min(TMS, S - j * TMS));
+        if (tid < E) {
+            for (uint32_t k = 0; k < sfull; ++k) put(ssh + (t0s >> 16) + k, tid, f + k * TMS, TMS);
+            if (srem) put(atomicAdd(&sbin[srem], 1u), tid, f + sfull * TMS, srem);
+        }
+        for (uint32_t t = nst + tid; t < scap; t += 1024u) put(t, 0u, 0u, 0u);
+    }
+    const uint32_t ntiles = min(nsh + nfull_all + nt_all, cap);
     for (uint32_t j = tid; j < nsh && j < cap; j += 1024u) {
         uint32_t* tl = tiles + 4u * j;
         tl[0] = E;
@@ -1694,7 +1716,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
             }
         }
     }
-    for (uint32_t t = nsh + tot[1] + nt_all + tid; t < cap; t += 1024u) {
+    for (uint32_t t = nsh + nfull_all + nt_all + tid; t < cap; t += 1024u) {
         uint32_t* tl = tiles + 4u * t;
         tl[0] = tl[1] = tl[2] = 0;
         tl[3] = ntiles;
@@ -2094,57 +2116,21 @@ __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15u) | ((N >> 4) << 14));
 }
 
-// Grouped GEMM on f16 MFMA for Q4_K, IQ3_XXS and IQ4_NL weights (see the
-// block comment above). e_shared names the tile expert id whose weights are
-// ws0/ws1 (the shared expert, run in the same launch); no tile carries it when
-// it is 0xffffffff. AORD (gate/up only) is the column order in which act is
-// stored: the order the down projection's format reads (a_pos).
-//   Pipeline. A slabs go straight from L2 to LDS (buffer_load ... lds; lane i
-// of a load writes 16 bytes at M0 + 16 i), two buffers by slab parity, so A
-// takes no registers. Per slab s: barrier; A(s + 1) into the other buffer, the
-// B ring's loads, at a superblock's first slab the next header (these loads
-// kept together and in this order); MFMAs of slab s with the operands decoded
-// one slab earlier, and the decode of slab s + 1 (into a second operand set,
-// interleaved with the MFMAs, when the tile has at most two row blocks; after
-// them otherwise); at a superblock's end the mins and the unit change; then a
-// wait for this wave's A(s + 1) only (vector-memory loads complete in issue
-// order, so vmcnt counts the B loads issued after it), which the next barrier
-// publishes. Every A DMA has landed before the block exits.
-//   TT (tile tokens) 64: 2 waves; wave w owns B rows (gate/up: gate and up rows
-// 32 w .. + 31 of the block's 64; down: rows 64 w .. + 63 of its 128) for all
-// 64 tokens, as 4 x 4 MFMA tiles. TT 128 (tiles of up to 128 pairs, for
-// batches in which an expert can take more than 64): 4 waves; wave w owns
-// gate and up rows 16 w .. + 15 (down: rows 32 w .. + 31) for all 128 tokens,
-// as 8 x 2 MFMA tiles. Each decoded B fragment then feeds 16 MFMAs instead of
-// 8 and each weight byte is fetched once per 128 tokens instead of 64; the A
-// slab (128 rows) is shared by the 4 waves through LDS.
-//   TL: the weights are in the tiled layout of k_tile_weights, where each B
-// load instruction reads one contiguous span
-// (every lane the bytes it decodes) instead of 16 rows' scattered pieces.
-template <int KIND, bool GATEUP, int AORD, int TT, bool TL = false>
-__global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_f16(
-    const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const uint8_t* __restrict__ ws0,
-    const uint8_t* __restrict__ ws1, uint32_t e_shared, uint64_t stride0, uint64_t stride1, uint32_t rows_per_expert,
-    uint32_t kdim, const _Float16* __restrict__ ah, const _Float16* __restrict__ al, const float* __restrict__ gs,
-    const uint32_t* __restrict__ pairs, uint32_t K, const uint32_t* __restrict__ tiles, uint32_t ldo, float limit,
-    float* __restrict__ out, _Float16* __restrict__ out_h, _Float16* __restrict__ out_l, float* __restrict__ out_gs,
-    uint32_t nblk, uint32_t a_rows, const float* __restrict__ xstat, uint32_t* __restrict__ rowmax,
-    uint32_t* __restrict__ flags, const uint32_t* __restrict__ slot_of) {
-    static_assert(KIND == 12 || KIND == 13 || KIND == 14 || KIND == 17 || KIND == 18 || KIND == 20 || KIND == 21 ||
-                      KIND == 22 || KIND == 23,
-                  "f16 GEMM formats: Q4_K, Q5_K, Q6_K, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_NL, IQ4_XS");
-    static_assert(AORD == A_NATURAL || GATEUP, "the permuted act layout is written by the gate/up kernel");
-    static_assert(TT == 64 || TT == 128, "tiles of 64 or 128 tokens");
-    // NB: 16-row B blocks per wave (gate/up: HB = NB / 2 gate, HB up); NW waves.
-    constexpr int NB = TT == 128 ? 2 : 4;
-    constexpr uint32_t NW = TT / 32u, HB = NB / 2;
+// The B operands of one wave of the f16 GEMMs: NB row blocks of 16 weight rows
+// (GATEUP: the first half gate rows, the second the same up rows), read as GGUF
+// bytes (TL: in the tiled layout) and decoded to exact f16 integers slab by slab.
+// load_hdr and load_slab issue a superblock's and a slab's loads (the slab's into
+// ring slot rs), take_hdr and decode turn them into scales and operands.
+template <int KIND, int NB, bool GATEUP, bool TL>
+struct BStream {
+    static constexpr int HB = NB / 2;
     // Q5_K is Q4_K with a fifth bit per value (b[16 + k % 32] bit k / 32 of its
     // superblock, kernels/iq3_mix.metal:19-23): the same header, scales, mins
     // and operand build, nibbles 32 bytes later in a 176-byte superblock, and
     // a lane's 8 fifth-bit bytes (the same byte positions as its nibble bytes,
     // bits 2 sq and 2 sq + 1 for slab sq) loaded with each header. q * sc is at
     // most 31 * 63 = 1953, an exact f16 integer as for Q4_K.
-    constexpr bool Q5K = KIND == 13, Q4K = KIND == 12 || Q5K, IQ3 = KIND == 18, IQ4 = KIND == 20;
+    static constexpr bool Q5K = KIND == 13, Q4K = KIND == 12 || Q5K, IQ3 = KIND == 18, IQ4 = KIND == 20;
     // IQ2_XS takes IQ3_XXS's path: 74-byte superblocks (2 bytes off a dword
     // every other one, like 98), lane kq's 16 bytes of 9+7-bit codes at
     // 2 + 16 kq (8 codes: 64 columns, two per slab, in A_IQ3XXS order), all 8
@@ -2159,12 +2145,12 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     // of the 512-entry grid), the ninth index bit from qh[2 kq], qh[2 kq + 1]
     // (66), its 8 sign bytes at 74 + 8 kq, the scale byte 106 + kq (a nibble per
     // 32-value group). B = (1 + 2 s) * grid * sign <= 31 * 15, unit d * 2^24.
-    constexpr bool IQ2 = KIND == 17, IQ2S = KIND == 22, IQ3S = KIND == 21, IQG = IQ2 || IQ2S || IQ3 || IQ3S;
+    static constexpr bool IQ2 = KIND == 17, IQ2S = KIND == 22, IQ3S = KIND == 21, IQG = IQ2 || IQ2S || IQ3 || IQ3S;
     // IQ4_XS takes IQ4_NL's path (B = the codebook value, a unit per 32-column
     // block): its blocks' 16 quant bytes sit at 8 + 16 g of a 136-byte
     // superblock (dword aligned), and a block's unit is d * (scale - 32), the
     // 6-bit scale from the 8-byte superblock header read with each slab.
-    constexpr bool IQ4X = KIND == 23, IQN = IQ4 || IQ4X;
+    static constexpr bool IQ4X = KIND == 23, IQN = IQ4 || IQ4X;
     // Q6_K (210-byte superblocks, kernels/moe.metal:22-28): w = d sc (q - 32),
     // q = 4 bits of ql | 2 bits of qh, sc an int8 per 16 columns; |sc (q - 32)|
     // reaches 4096, past the 2048 that f16 holds exactly, so B enters twice:
@@ -2181,136 +2167,28 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     // take the dword-aligned window and shift by 16 bits where it does (no
     // byte it uses sits in a dword past its superblock), and d comes from a
     // 16-bit load.
-    constexpr bool Q6K = KIND == 14;
-    // (two operand sets per fragment: TT 128's 2 row blocks per wave fit the registers, 4 do not)
-    static_assert(!Q6K || TT == 128, "Q6_K runs on 128-token tiles (which also take tiles of 64)");
-    constexpr uint32_t IQB = IQ2 ? 74u : IQ2S ? 82u : IQ3S ? 110u : Q6K ? 210u : 98u;
-    constexpr uint32_t SBB = Q5K ? 176u : 144u, QOFF = Q5K ? 48u : 16u;
+    static constexpr bool Q6K = KIND == 14;
+    static constexpr uint32_t IQB = IQ2 ? 74u : IQ2S ? 82u : IQ3S ? 110u : Q6K ? 210u : 98u;
+    static constexpr uint32_t SBB = Q5K ? 176u : 144u, QOFF = Q5K ? 48u : 16u;
     // tiled record bytes (per superblock; IQ4_NL: per slab)
-    constexpr uint32_t TREC = tile_record(KIND);
-    constexpr uint32_t UNR = 4u;
-    // A slab buffers (hi, lo; by slab parity): 64 halves (128 B) per token row,
-    // 16-byte chunk c of row r at slot c ^ ((r >> 1) & 7), so that the fragment
-    // reads (16 rows at one chunk) touch every bank once. Separate objects, so
-    // that the compiler sees that a DMA into one never aliases reads of the
-    // other. S tiles (Q4_K group sums) by superblock parity.
-    __shared__ _Float16 Ah0[TT * 64], Ah1[TT * 64], Al0[TT * 64], Al1[TT * 64];
-    __shared__ _Float16 Ss[2][TT * 16];  // per row: S hi of groups 0..7, S lo of groups 0..7
-    // Tile rounds of 8 (one tile per XCD) alternate direction: XCD x takes tile
-    // 8 ti + x in even rounds and 8 ti + 7 - x in odd ones. The tiles come
-    // sorted by decreasing size, so a fixed direction would give XCD 0 the
-    // largest tile of every round (a dispatch simulation over C1's tiles with
-    // measured block times: XCD spans 62-85 us against 70-76 us snaked;
-    // measured: C1 gate/up about 1.4 us shorter, C3 gate/up 176-178 to
-    // 169-170 us, C3 down 114-116 to 111-113).
-    const uint32_t nt = tiles[3], slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
-    const uint32_t t = ti * 8u + ((ti & 1u) ? 7u - xcd : xcd);
-    if (t >= nt) return;
-    const uint32_t* tile = tiles + 4u * t;
-    const uint32_t n = tile[2];
-    if (n == 0) return;
-    // Cached experts (slot_of != NULL, entry E for the shared expert's tiles):
-    // the expert's weights are in slot slot_of[e], or it is not resident in this
-    // pass (NO_SLOT) and the tile waits for a later one.
-    const uint32_t ew = slot_of ? slot_of[tile[0]] : tile[0];
-    if (ew == NO_SLOT) return;
-    if constexpr (!Q4K && !Q6K) {
-        stage_f16_tables<KIND>();
-        __syncthreads();
-    }
-    const uint32_t e = tile[0], q0 = tile[1];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, ln = lane & 15u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t row0 = (slot - ti * nblk) * (GATEUP ? 64u : 128u);
-    const uint32_t ngroups = kdim / 32u;
+    static constexpr uint32_t TREC = tile_record(KIND);
 
-    // A DMA: instruction i of wave w fills tile rows 8 (NW i + w) .. + 7; lane l
-    // writes row r = 8 (NW i + w) + l / 8 at LDS slot l % 8, which holds chunk
-    // (l % 8) ^ ((r >> 1) & 7) of the row (the swizzle of the fragment reads).
-    uint32_t avo[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t r = 8u * (NW * i + wave) + (lane >> 3);
-        const uint32_t q = q0 + (r < n ? r : 0u);
-        const uint32_t arow = GATEUP ? (pairs ? pairs[q] / K : q) : q;
-        avo[i] = 2u * (arow * kdim + 8u * ((lane & 7u) ^ ((r >> 1) & 7u)));
-    }
-    const uint32_t am = tid >> 1, ahalf = tid & 1u;
-    uint32_t soff = 0;
-    if constexpr (Q4K) {
-        const uint32_t q = q0 + (am < n ? am : 0u);
-        const uint32_t r = GATEUP ? (pairs ? pairs[q] / K : q) : q;
-        soff = 4u * (r * ngroups + 4u * ahalf);
-    }
-    // GATEUP: the split exponent e_t of each tile row's token and the units
-    // exponent a_t of its activations, for the epilogue (published by the main
-    // loop's first barrier). Down: row block 0 of each tile checks that its
-    // activation rows were split in range.
-    __shared__ int2 s_rowe[TT];
-    // TT 128 gate/up: each wave's 16-column halves of the act group sums
-    __shared__ float gpart[GATEUP && TT == 128 ? 4 : 1][TT];
-    // gate/up: each wave's maximum of |act| over its columns of a row, reduced
-    // over the NW waves before one atomicMax per row and block (one per wave
-    // before: C1 gate/up 86.2-86.6 to 81.9-85.7 us, the Q4_K/Q6_K mix at 512
-    // tokens 111.8-114.3 to 101.6-105.1)
-    __shared__ uint32_t rpart[GATEUP ? NW : 1][TT];
-    if constexpr (GATEUP) {
-        if (tid < TT) {
-            const uint32_t q = q0 + (tid < n ? tid : 0u);
-            const float2 st = ld_xstat(xstat, pairs ? pairs[q] / K : q);
-            s_rowe[tid] = make_int2(x_exp(st.x), act_exp(st));
-        }
-    } else {
-        if (rowmax != nullptr && slot - ti * nblk == 0u) {
-            bool bad = false;
-            if (tid < n) {
-                const float m = __uint_as_float(rowmax[q0 + tid]);
-                bad = !(m == 0.f || (m >= ACT_RANGE_LO && m < ACT_RANGE_HI));  // NaN: bad
-            }
-            if (__any(bad) && lane == 0u) atomicOr(flags, FLAG_RANGE);
-        }
-    }
-    const bool sh_tile = e == e_shared;
-    const uint8_t* const wb0 = sh_tile ? ws0 : w0 + (uint64_t)ew * rows_per_expert * stride0;
-    const uint8_t* const wb1 = GATEUP ? (sh_tile ? ws1 : w1 + (uint64_t)ew * rows_per_expert * stride1) : wb0;
-    const __amdgpu_buffer_rsrc_t ra_h = make_rsrc(ah, (uint32_t)(kdim * 2u) * a_rows);
-    const __amdgpu_buffer_rsrc_t ra_l = make_rsrc(al, (uint32_t)(kdim * 2u) * a_rows);
-    const __amdgpu_buffer_rsrc_t rgs = make_rsrc(gs, ngroups * 4u * a_rows);
-    const __amdgpu_buffer_rsrc_t rw0 = make_rsrc(wb0, (uint32_t)(rows_per_expert * stride0));
-    const __amdgpu_buffer_rsrc_t rw1 = GATEUP ? make_rsrc(wb1, (uint32_t)(rows_per_expert * stride1)) : rw0;
-    uint32_t bsoff[NB], boff[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-        if (GATEUP) {
-            const uint32_t st = (uint32_t)(nb < (int)HB ? stride0 : stride1);
-            bsoff[nb] = (row0 + 16u * HB * wave + 16u * (nb % HB)) * st;
-            boff[nb] = ln * st;
-        } else {
-            bsoff[nb] = (row0 + 16u * NB * wave + 16u * nb) * (uint32_t)stride0;
-            boff[nb] = ln * (uint32_t)stride0;
-        }
-    }
-    const uint32_t slabs = kdim / 64u, sbs = kdim / 256u;
-    // Q6_K: each lane's row start (bytes from the expert's base)
-    uint32_t q6r[Q6K ? NB : 1];
-    if constexpr (Q6K) {
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) q6r[nb] = bsoff[nb] + boff[nb];
-    }
+    __amdgpu_buffer_rsrc_t rw0, rw1;
+    uint32_t bsoff[NB], boff[NB];  // per row block: its first row's byte (uniform), the lane's row within it
+    uint32_t slabs, sbs, lane, kq, ln;
+    uint32_t q6r[Q6K ? NB : 1];  // Q6_K: each lane's row start (bytes from the expert's base)
 
-    float4 ps;
-#define INGOT_LOAD_S(SB) ps = __builtin_bit_cast(float4, buf_load16(rgs, soff, 32u * ((SB) < sbs ? (SB) : sbs - 1u)))
     uint4 nhdr[NB];
     uint2 nqh[Q5K ? NB : 1];
     uint32_t n5[NB], n_d[NB];
     uint3 n3[NB], ns3[IQ2S ? NB : 1];
     uint4 nqh3[IQ3S ? NB : 1];  // IQ3_S: bytes 64 .. 79 (qh) and 104 .. 111 (scales) of the superblock's dword window
     uint2 nsc3[IQ3S ? NB : 1];
-    auto load_hdr = [&](uint32_t sb) {
+    __device__ __forceinline__ void load_hdr(uint32_t sb) {
         sb = sb < sbs ? sb : sbs - 1u;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const __amdgpu_buffer_rsrc_t rw = GATEUP && nb >= (int)HB ? rw1 : rw0;
+            const __amdgpu_buffer_rsrc_t rw = GATEUP && nb >= HB ? rw1 : rw0;
             if constexpr (TL && Q4K) nhdr[nb] = buf_load16(rw, 16u * ln, bsoff[nb] + sb * TREC);
             else if constexpr (Q4K) nhdr[nb] = buf_load16(rw, boff[nb], bsoff[nb] + sb * SBB);
             if constexpr (TL && Q5K) nqh[nb] = buf_load8(rw, 8u * lane, bsoff[nb] + sb * TREC + 256u);
@@ -2378,17 +2256,17 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 n_d[nb] = __builtin_amdgcn_raw_buffer_load_b16(rw, (int)b, 208, 0);
             }
         }
-    };
+    }
     uint4 nq[4][NB];
     uint32_t n1[4][NB];
     uint2 nd[4][NB];
     // Q6_K: ev (the slab is the first of its half, a compile-time constant at
     // each call) also loads the half's qh window.
-    auto load_slab = [&](uint32_t rs, uint32_t s, bool ev = false) {
+    __device__ __forceinline__ void load_slab(uint32_t rs, uint32_t s, bool ev = false) {
         s = s < slabs ? s : slabs - 1u;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            const __amdgpu_buffer_rsrc_t rw = GATEUP && nb >= (int)HB ? rw1 : rw0;
+            const __amdgpu_buffer_rsrc_t rw = GATEUP && nb >= HB ? rw1 : rw0;
             if constexpr (TL && Q6K) {
                 // ql bytes of the slab, and at a half's first slab its qh bytes
                 const uint32_t u = bsoff[nb] + (s >> 2) * TREC, hn = (s >> 1) & 1u;
@@ -2449,18 +2327,18 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 nd[rs][nb] = make_uint2(buf_load4(rw, boff[nb], u), buf_load4(rw, boff[nb], u + 16u));
             }
         }
-    };
-    auto dbits = [&](int nb, uint32_t sb) -> uint32_t {
+    }
+    __device__ __forceinline__ uint32_t dbits(int nb, uint32_t sb) const {
         if constexpr (TL && IQG) return (ln & 1u) ? n_d[nb] >> 16 : n_d[nb];
         if constexpr (IQG) return (sb & 1u) ? n_d[nb] >> 16 : n_d[nb];
         if constexpr (TL && Q6K) return ((ln & 1u) ? n_d[nb] >> 16 : n_d[nb]) & 0xffffu;
         if constexpr (Q6K) return n_d[nb];
         return nhdr[nb].x;
-    };
-    auto unit = [](uint32_t bits) {
+    }
+    static __device__ __forceinline__ float unit(uint32_t bits) {
         const float d = half_bits_to_float(bits);
         return d != 0.f ? d * ((IQ2 || IQ2S) ? 2097152.f : IQ3 ? 4194304.f : Q6K ? 1.f : 16777216.f) : 1.f;
-    };
+    }
     // Superblock state for the decode (and, at the superblock's end, the mins
     // and the unit change).
     struct SbState {
@@ -2470,7 +2348,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
         float dsc[NB], dmn[NB];
         uint32_t sh[Q6K ? NB : 1];  // Q6_K: the lane's superblock misalignment in bits (0 or 16)
     };
-    auto take_hdr = [&](SbState& st, uint32_t sb) {
+    __device__ __forceinline__ void take_hdr(SbState& st, uint32_t sb) const {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             const uint32_t db = dbits(nb, sb);
@@ -2559,17 +2437,17 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 for (int i = 0; i < 4; ++i) st.gw[nb][i] = z ? 0u : __builtin_amdgcn_alignbit(w[i + 1], w[i], st.sh[nb]);
             }
         }
-    };
+    }
     // Q6_K: the qh words of the half being decoded (set at its first slab), and
     // the perm selector of the lane's two scale bytes (byte kq / 2 of scale
     // words 2 n, 2 n + 1; + 2 in a half's second slab).
     uint2 qhc[Q6K ? NB : 1];
-    const uint32_t q6sel = 0x0c040c00u + (kq >> 1) * 0x00010001u;
+    uint32_t q6sel;
     // Decode of slab position sq (within its superblock) into fb (Q6_K: B_r
     // into fb, B_e into fe); IQ4_NL also yields the units of its two blocks and
     // whether a d is zero.
-    auto decode = [&](const SbState& st, uint32_t sq, const uint4* qv, const uint2* dv, half8 (*fb)[2],
-                      float (*dg)[2], half8 (*fe)[2]) {
+    __device__ __forceinline__ void decode(const SbState& st, uint32_t sq, const uint4* qv, const uint2* dv,
+                                           half8 (*fb)[2], float (*dg)[2], half8 (*fe)[2]) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             if constexpr (Q6K) {
@@ -2718,8 +2596,173 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 dg[nb][1] = d1 != 0.f ? d1 * 16777216.f : 1.f;
             }
         }
-    };
+    }
 
+    // wb0, wb1: the expert's matrices of `rows` rows; r0: the wave's first gate
+    // row and up row (down: its first row).
+    __device__ __forceinline__ void init(const uint8_t* wb0, const uint8_t* wb1, uint64_t stride0, uint64_t stride1,
+                                         uint32_t rows, uint32_t kdim, uint32_t r0, uint32_t lane_) {
+        lane = lane_;
+        kq = lane >> 4;
+        ln = lane & 15u;
+        slabs = kdim / 64u;
+        sbs = kdim / 256u;
+        q6sel = 0x0c040c00u + (kq >> 1) * 0x00010001u;
+        rw0 = make_rsrc(wb0, (uint32_t)(rows * stride0));
+        rw1 = GATEUP ? make_rsrc(wb1, (uint32_t)(rows * stride1)) : rw0;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const uint32_t st = (uint32_t)(!GATEUP || nb < HB ? stride0 : stride1);
+            bsoff[nb] = (r0 + 16u * (uint32_t)(GATEUP ? nb % HB : nb)) * st;
+            boff[nb] = ln * st;
+            if constexpr (Q6K) q6r[nb] = bsoff[nb] + boff[nb];
+        }
+    }
+};
+
+// Grouped GEMM on f16 MFMA for Q4_K, IQ3_XXS and IQ4_NL weights (see the
+// block comment above). e_shared names the tile expert id whose weights are
+// ws0/ws1 (the shared expert, run in the same launch); no tile carries it when
+// it is 0xffffffff. AORD (gate/up only) is the column order in which act is
+// stored: the order the down projection's format reads (a_pos).
+//   Pipeline. A slabs go straight from L2 to LDS (buffer_load ... lds; lane i
+// of a load writes 16 bytes at M0 + 16 i), two buffers by slab parity, so A
+// takes no registers. Per slab s: barrier; A(s + 1) into the other buffer, the
+// B ring's loads, at a superblock's first slab the next header (these loads
+// kept together and in this order); MFMAs of slab s with the operands decoded
+// one slab earlier, and the decode of slab s + 1 (into a second operand set,
+// interleaved with the MFMAs, when the tile has at most two row blocks; after
+// them otherwise); at a superblock's end the mins and the unit change; then a
+// wait for this wave's A(s + 1) only (vector-memory loads complete in issue
+// order, so vmcnt counts the B loads issued after it), which the next barrier
+// publishes. Every A DMA has landed before the block exits.
+//   TT (tile tokens) 64: 2 waves; wave w owns B rows (gate/up: gate and up rows
+// 32 w .. + 31 of the block's 64; down: rows 64 w .. + 63 of its 128) for all
+// 64 tokens, as 4 x 4 MFMA tiles. TT 128 (tiles of up to 128 pairs, for
+// batches in which an expert can take more than 64): 4 waves; wave w owns
+// gate and up rows 16 w .. + 15 (down: rows 32 w .. + 31) for all 128 tokens,
+// as 8 x 2 MFMA tiles. Each decoded B fragment then feeds 16 MFMAs instead of
+// 8 and each weight byte is fetched once per 128 tokens instead of 64; the A
+// slab (128 rows) is shared by the 4 waves through LDS.
+//   TL: the weights are in the tiled layout of k_tile_weights, where each B
+// load instruction reads one contiguous span
+// (every lane the bytes it decodes) instead of 16 rows' scattered pieces.
+template <int KIND, bool GATEUP, int AORD, int TT, bool TL = false>
+__global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_f16(
+    const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const uint8_t* __restrict__ ws0,
+    const uint8_t* __restrict__ ws1, uint32_t e_shared, uint64_t stride0, uint64_t stride1, uint32_t rows_per_expert,
+    uint32_t kdim, const _Float16* __restrict__ ah, const _Float16* __restrict__ al, const float* __restrict__ gs,
+    const uint32_t* __restrict__ pairs, uint32_t K, const uint32_t* __restrict__ tiles, uint32_t ldo, float limit,
+    float* __restrict__ out, _Float16* __restrict__ out_h, _Float16* __restrict__ out_l, float* __restrict__ out_gs,
+    uint32_t nblk, uint32_t a_rows, const float* __restrict__ xstat, uint32_t* __restrict__ rowmax,
+    uint32_t* __restrict__ flags, const uint32_t* __restrict__ slot_of) {
+    static_assert(KIND == 12 || KIND == 13 || KIND == 14 || KIND == 17 || KIND == 18 || KIND == 20 || KIND == 21 ||
+                      KIND == 22 || KIND == 23,
+                  "f16 GEMM formats: Q4_K, Q5_K, Q6_K, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_NL, IQ4_XS");
+    static_assert(AORD == A_NATURAL || GATEUP, "the permuted act layout is written by the gate/up kernel");
+    static_assert(TT == 64 || TT == 128, "tiles of 64 or 128 tokens");
+    // NB: 16-row B blocks per wave (gate/up: HB = NB / 2 gate, HB up); NW waves.
+    constexpr int NB = TT == 128 ? 2 : 4;
+    constexpr uint32_t NW = TT / 32u, HB = NB / 2;
+    using BS = BStream<KIND, NB, GATEUP, TL>;
+    constexpr bool Q5K = BS::Q5K, Q4K = BS::Q4K, IQ2S = BS::IQ2S, IQ3S = BS::IQ3S, IQG = BS::IQG, IQ4 = BS::IQ4,
+                   IQ4X = BS::IQ4X, IQN = BS::IQN, Q6K = BS::Q6K;
+    // (two operand sets per fragment: TT 128's 2 row blocks per wave fit the registers, 4 do not)
+    static_assert(!Q6K || TT == 128, "Q6_K runs on 128-token tiles (which also take tiles of 64)");
+    constexpr uint32_t UNR = 4u;
+    // A slab buffers (hi, lo; by slab parity): 64 halves (128 B) per token row,
+    // 16-byte chunk c of row r at slot c ^ ((r >> 1) & 7), so that the fragment
+    // reads (16 rows at one chunk) touch every bank once. Separate objects, so
+    // that the compiler sees that a DMA into one never aliases reads of the
+    // other. S tiles (Q4_K group sums) by superblock parity.
+    __shared__ _Float16 Ah0[TT * 64], Ah1[TT * 64], Al0[TT * 64], Al1[TT * 64];
+    __shared__ _Float16 Ss[2][TT * 16];  // per row: S hi of groups 0..7, S lo of groups 0..7
+    // Tile rounds of 8 (one tile per XCD) alternate direction: XCD x takes tile
+    // 8 ti + x in even rounds and 8 ti + 7 - x in odd ones. The tiles come
+    // sorted by decreasing size, so a fixed direction would give XCD 0 the
+    // largest tile of every round (a dispatch simulation over C1's tiles with
+    // measured block times: XCD spans 62-85 us against 70-76 us snaked;
+    // measured: C1 gate/up about 1.4 us shorter, C3 gate/up 176-178 to
+    // 169-170 us, C3 down 114-116 to 111-113).
+    const uint32_t nt = tiles[3], slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
+    const uint32_t t = ti * 8u + ((ti & 1u) ? 7u - xcd : xcd);
+    if (t >= nt) return;
+    const uint32_t* tile = tiles + 4u * t;
+    const uint32_t n = tile[2];
+    if (n == 0) return;
+    // Cached experts (slot_of != NULL, entry E for the shared expert's tiles):
+    // the expert's weights are in slot slot_of[e], or it is not resident in this
+    // pass (NO_SLOT) and the tile waits for a later one.
+    const uint32_t ew = slot_of ? slot_of[tile[0]] : tile[0];
+    if (ew == NO_SLOT) return;
+    if constexpr (!Q4K && !Q6K) {
+        stage_f16_tables<KIND>();
+        __syncthreads();
+    }
+    const uint32_t e = tile[0], q0 = tile[1];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, ln = lane & 15u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t row0 = (slot - ti * nblk) * (GATEUP ? 64u : 128u);
+    const uint32_t ngroups = kdim / 32u;
+
+    // A DMA: instruction i of wave w fills tile rows 8 (NW i + w) .. + 7; lane l
+    // writes row r = 8 (NW i + w) + l / 8 at LDS slot l % 8, which holds chunk
+    // (l % 8) ^ ((r >> 1) & 7) of the row (the swizzle of the fragment reads).
+    uint32_t avo[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t r = 8u * (NW * i + wave) + (lane >> 3);
+        const uint32_t q = q0 + (r < n ? r : 0u);
+        const uint32_t arow = GATEUP ? (pairs ? pairs[q] / K : q) : q;
+        avo[i] = 2u * (arow * kdim + 8u * ((lane & 7u) ^ ((r >> 1) & 7u)));
+    }
+    const uint32_t am = tid >> 1, ahalf = tid & 1u;
+    uint32_t soff = 0;
+    if constexpr (Q4K) {
+        const uint32_t q = q0 + (am < n ? am : 0u);
+        const uint32_t r = GATEUP ? (pairs ? pairs[q] / K : q) : q;
+        soff = 4u * (r * ngroups + 4u * ahalf);
+    }
+    // GATEUP: the split exponent e_t of each tile row's token and the units
+    // exponent a_t of its activations, for the epilogue (published by the main
+    // loop's first barrier). Down: row block 0 of each tile checks that its
+    // activation rows were split in range.
+    __shared__ int2 s_rowe[TT];
+    // TT 128 gate/up: each wave's 16-column halves of the act group sums
+    __shared__ float gpart[GATEUP && TT == 128 ? 4 : 1][TT];
+    // gate/up: each wave's maximum of |act| over its columns of a row, reduced
+    // over the NW waves before one atomicMax per row and block (one per wave
+    // before: C1 gate/up 86.2-86.6 to 81.9-85.7 us, the Q4_K/Q6_K mix at 512
+    // tokens 111.8-114.3 to 101.6-105.1)
+    __shared__ uint32_t rpart[GATEUP ? NW : 1][TT];
+    if constexpr (GATEUP) {
+        if (tid < TT) {
+            const uint32_t q = q0 + (tid < n ? tid : 0u);
+            const float2 st = ld_xstat(xstat, pairs ? pairs[q] / K : q);
+            s_rowe[tid] = make_int2(x_exp(st.x), act_exp(st));
+        }
+    } else {
+        if (rowmax != nullptr && slot - ti * nblk == 0u) {
+            bool bad = false;
+            if (tid < n) {
+                const float m = __uint_as_float(rowmax[q0 + tid]);
+                bad = !(m == 0.f || (m >= ACT_RANGE_LO && m < ACT_RANGE_HI));  // NaN: bad
+            }
+            if (__any(bad) && lane == 0u) atomicOr(flags, FLAG_RANGE);
+        }
+    }
+    const bool sh_tile = e == e_shared;
+    const uint8_t* const wb0 = sh_tile ? ws0 : w0 + (uint64_t)ew * rows_per_expert * stride0;
+    const uint8_t* const wb1 = GATEUP ? (sh_tile ? ws1 : w1 + (uint64_t)ew * rows_per_expert * stride1) : wb0;
+    const __amdgpu_buffer_rsrc_t ra_h = make_rsrc(ah, (uint32_t)(kdim * 2u) * a_rows);
+    const __amdgpu_buffer_rsrc_t ra_l = make_rsrc(al, (uint32_t)(kdim * 2u) * a_rows);
+    const __amdgpu_buffer_rsrc_t rgs = make_rsrc(gs, ngroups * 4u * a_rows);
+    BS B;
+    B.init(wb0, wb1, stride0, stride1, rows_per_expert, kdim, row0 + 16u * (GATEUP ? HB : NB) * wave, lane);
+    const uint32_t slabs = B.slabs, sbs = B.sbs;
+
+    float4 ps;
+#define INGOT_LOAD_S(SB) ps = __builtin_bit_cast(float4, buf_load16(rgs, soff, 32u * ((SB) < sbs ? (SB) : sbs - 1u)))
     // Q4_K group sums of this thread's row divided by 32 (exact; they reach
     // 2^16 for x and 2^19 for act within range), split hi/lo, into an S buffer.
     auto store_s = [&](_Float16* sb_) {
@@ -2770,15 +2813,15 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
             for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
         // Prologue: A(0) into buffer 0; B ring; header of superblock 0; decode B(0).
         dma_a(0u, 0u);
-        if constexpr (!IQN) load_hdr(0);
+        if constexpr (!IQN) B.load_hdr(0);
         if constexpr (Q4K) {
             INGOT_LOAD_S(0u);
             store_s(Ss[0]);
         }
 #pragma unroll
-        for (uint32_t d = 0; d < DEPTH; ++d) load_slab(d, d, (d & 1u) == 0u);
-        SbState cur, nxt;
-        if constexpr (!IQN) take_hdr(cur, 0u);
+        for (uint32_t d = 0; d < DEPTH; ++d) B.load_slab(d, d, (d & 1u) == 0u);
+        typename BS::SbState cur, nxt;
+        if constexpr (!IQN) B.take_hdr(cur, 0u);
         half8 fb[NFB][NB][2], fe[Q6K ? NFB : 1][NB][2];
         float dgs[NFB][NB][2];
         {
@@ -2786,12 +2829,12 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
             uint2 dv[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                qv[nb] = nq[0][nb];
-                if constexpr (IQN) qv[nb].z = n1[0][nb];
-                if constexpr (IQN || Q6K) dv[nb] = nd[0][nb];
+                qv[nb] = B.nq[0][nb];
+                if constexpr (IQN) qv[nb].z = B.n1[0][nb];
+                if constexpr (IQN || Q6K) dv[nb] = B.nd[0][nb];
             }
-            load_slab(0, DEPTH, true);
-            decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0]);
+            B.load_slab(0, DEPTH, true);
+            B.decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0]);
         }
         for (uint32_t s0 = 0; s0 < slabs; s0 += UNR) {
             const uint32_t sb = s0 >> 2;
@@ -2817,28 +2860,28 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 uint2 dv[NB];
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
-                    qv[nb] = nq[rs][nb];
-                    if constexpr (IQN) qv[nb].z = n1[rs][nb];
-                    if constexpr (IQN || Q6K) dv[nb] = nd[rs][nb];
+                    qv[nb] = B.nq[rs][nb];
+                    if constexpr (IQN) qv[nb].z = B.n1[rs][nb];
+                    if constexpr (IQN || Q6K) dv[nb] = B.nd[rs][nb];
                 }
                 // (s is a multiple of UNR plus sq: slab s + 1 + DEPTH opens a half when sq is odd)
-                load_slab(rs, s + 1u + DEPTH, (sq & 1u) != 0u);
+                B.load_slab(rs, s + 1u + DEPTH, (sq & 1u) != 0u);
                 if constexpr (!IQN) {
                     if (sq == 0) {
-                        load_hdr(sb + 1);
+                        B.load_hdr(sb + 1);
                         if constexpr (Q4K) INGOT_LOAD_S(sb + 1u);
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if constexpr (!IQN) {
                     // past the last superblock: the clamped header, never used
-                    if (sq == 3) take_hdr(nxt, sb + 1u);
+                    if (sq == 3) B.take_hdr(nxt, sb + 1u);
                 }
                 // Decode B(s + 1) while this slab's MFMAs issue.
                 const uint32_t cb = NFB == 2u ? (sq & 1u) : 0u, nb_ = NFB == 2u ? cb ^ 1u : 0u;
                 // (after the last slab: a decode of clamped bytes that nothing reads;
                 // kept unconditional so that the decode shares a block with the MFMAs)
-                if (NFB == 2u) decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u]);
+                if (NFB == 2u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u]);
                 const _Float16* const bh = (sq & 1u) ? Ah1 : Ah0;
                 const _Float16* const bl = (sq & 1u) ? Al1 : Al0;
                 if constexpr (!IQN) {
@@ -2915,7 +2958,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                             }
                     }
                 }
-                if (NFB == 1u) decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0]);
+                if (NFB == 1u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0]);
                 if constexpr (Q4K) {
                     if (sq == 3) {
                         half8 fm[NB];

@@ -1,0 +1,49 @@
+"""The grouped GEMM's two tile kernels at the sizes where they can go wrong:
+expert loads at the edges of the small-tile GEMM's operands (8 pairs packed hi
+and lo in one operand, 16 pairs per tile) and just past them, empty experts, a
+K that ends inside an A chunk, merged shared tiles; and the same loads doubled,
+past the rule that selects the small tiles (12 pairs per expert). Against the
+oracle, to the repository's bar; and GGUF-order weights (a cached layer) bit for
+bit against the tiled copies (a resident one)."""
+import numpy as np
+import pytest
+
+from ingot_amd import configs as CF
+from ingot_amd.moe import IQ2_S, IQ2_XS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q4_K, Q5_K, Q6_K, MoeLayer
+from util import check_layer
+
+pytestmark = pytest.mark.gpu
+
+LOADS = [1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 0, 5, 0, 0, 1, 2]  # 177 pairs, 11.1 per expert
+
+
+def routed_inputs(spec, loads, H, seed):
+    """Inputs whose identity router sends loads[e] tokens to expert e (top-1)."""
+    E = len(loads)
+    T = sum(loads)
+    spec.router = np.zeros((E, H), np.float32)
+    spec.router[np.arange(E), np.arange(E)] = 1.0
+    x = CF.inputs(seed, T, H) * 0.05
+    order = np.repeat(np.arange(E), loads)
+    np.random.default_rng(seed).shuffle(order)
+    x[:, :E] = 0.0
+    x[np.arange(T), order] = 4.0
+    return x
+
+
+@pytest.mark.parametrize("gk,dk,F", [(Q4_K, Q4_K, 256), (Q5_K, Q5_K, 768), (Q6_K, Q6_K, 256), (Q4_K, Q6_K, 768),
+                                     (IQ2_XS, IQ2_XS, 512), (IQ2_S, IQ2_S, 512), (IQ3_XXS, IQ4_NL, 192),
+                                     (IQ3_S, IQ3_S, 512), (IQ4_XS, IQ4_XS, 256), (IQ4_NL, IQ4_NL, 64)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_tile_loads(gpu, oracle, gk, dk, F, shared):
+    H, E = 1024, len(LOADS)
+    spec = CF.make_layer(61, 0, H, E, 1, F, gk, dk, shared_ffn=F if shared else 0)
+    for times in (1, 2):  # small tiles; past the rule
+        loads = [times * v for v in LOADS]
+        x = routed_inputs(spec, loads, H, 61 + times)
+        res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
+        out, ids, _ = check_layer(res, spec, x, oracle, f"{gk}/{dk} F={F} shared={shared} {times}x loads")
+        assert np.array_equal(np.bincount(ids.ravel(), minlength=E), loads)
+        assert np.array_equal(out, cached(x)[0]), "GGUF order against tiled copies"
+        res.destroy()
+        cached.destroy()
