@@ -288,7 +288,10 @@ int ingot_layer_forward_add(ingot_layer* layer, const float* d_x, const float* d
  * [2^10, 2^11)); when a row's max |act| so scaled leaves [2^-3, 2^14) (weights
  * far from the usual size) the forward raises the device flag that
  * ingot_ctx_check_device_flags reports as INGOT_RANGE, and its outputs must
- * be recomputed with INGOT_GEMM_FP32.
+ * be recomputed with INGOT_GEMM_FP32. Layers whose gate, up and down are all
+ * Q8_0 run on it too (B the int8 value, f16 hi + lo scaled by each activation
+ * row's own maximum, so without a range); beside another format a Q8_0
+ * projection keeps the fp32 GEMM.
  * INGOT_GEMM_FP32: always the fp32 MFMA GEMM. */
 enum ingot_gemm_mode { INGOT_GEMM_AUTO = 0, INGOT_GEMM_FP32 = 1 };
 int ingot_layer_set_gemm_mode(ingot_layer* layer, uint32_t mode);

@@ -15,7 +15,7 @@
 //     the lo rows in rows 8..15 of ONE operand (512 columns per chunk), so each
 //     decoded B fragment feeds one MFMA instead of two and the halves meet in
 //     the epilogue; tiles of 9..16 pairs hold hi and lo operands of 16 rows
-//     (256 columns per chunk);
+//     (256 columns per chunk; a superblock each measured 3 % slower packed);
 //   * each superblock is summed from zero and then added to the total times its
 //     unit (one fma per value), which needs no reciprocal of the next unit.
 // Gate/up + down, k_gemm_f16 against this kernel: a Qwen3-30B-A3B-shaped layer
@@ -28,8 +28,13 @@
 
 namespace ingot {
 
-template <int KIND, bool GATEUP, int AORD, bool TL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : KIND == 14 ? 3 : 4))) void k_gemm_small(
+// tiles == NULL: a dense product (a shared expert beside routed experts of
+// another format), tile t = rows 16 t .. of the a_rows input rows, expert 0.
+// XORD: the column order in which x is stored where it is not the order the
+// format reads (Q8_0's natural one): the operand's pieces are then looked up in
+// it, which every order that keeps runs of 8 columns inside a superblock allows.
+template <int KIND, bool GATEUP, int AORD, bool TL, int XORD = A_NATURAL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : KIND == 8 || KIND == 14 ? 3 : 4))) void k_gemm_small(
     const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const uint8_t* __restrict__ ws0,
     const uint8_t* __restrict__ ws1, uint32_t e_shared, uint64_t stride0, uint64_t stride1, uint32_t rows_per_expert,
     uint32_t kdim, const _Float16* __restrict__ ah, const _Float16* __restrict__ al, const float* __restrict__ gs,
@@ -41,7 +46,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
     constexpr int NB = 2;
     constexpr uint32_t NW = 4;
     using BS = BStream<KIND, NB, GATEUP, TL>;
-    constexpr bool Q4K = BS::Q4K, IQG = BS::IQG, IQN = BS::IQN, Q6K = BS::Q6K;
+    constexpr bool Q4K = BS::Q4K, IQG = BS::IQG, IQN = BS::IQN, Q6K = BS::Q6K, Q8 = BS::Q8;
+    static_assert(XORD == A_NATURAL || (Q8 && GATEUP && XORD != A_IQ4NL), "a natural operand in another order");
+    static_assert(!Q8 || !GATEUP || AORD == A_F32, "Q8_0 gate/up writes fp32 act (k_split_act)");
     __shared__ __align__(16) _Float16 As[2][8192];
     // Q4_K group sums / 32 of the chunk, f16: per superblock 16 rows x 8 groups
     // (packed: rows 0..7 the hi, 8..15 the lo parts) or 16 rows x {8 hi, 8 lo}
@@ -50,13 +57,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
     __shared__ float gpart[GATEUP ? NW : 1][TMS];
     __shared__ uint32_t rpart[GATEUP ? NW : 1][TMS];
     // tile rounds of 8, one tile per XCD, alternating direction (as k_gemm_f16)
-    const uint32_t nt = tiles[3], slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
+    const uint32_t nt = tiles ? tiles[3] : (a_rows + TMS - 1u) / TMS, slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
     const uint32_t t = ti * 8u + ((ti & 1u) ? 7u - xcd : xcd);
     if (t >= nt) return;
     const uint32_t* tile = tiles + 4u * t;
-    const uint32_t n = tile[2];
+    const uint32_t n = tiles ? tile[2] : min(TMS, a_rows - TMS * t);
     if (n == 0) return;
-    const uint32_t e = tile[0], q0 = tile[1];
+    const uint32_t e = tiles ? tile[0] : 0u, q0 = tiles ? tile[1] : TMS * t;
     const uint32_t ew = slot_of ? slot_of[e] : e;  // cached experts, as in k_gemm_f16
     if (ew == NO_SLOT) return;
     const uint32_t row0 = (slot - ti * nblk) * (GATEUP ? 64u : 128u);
@@ -68,7 +75,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
     const __amdgpu_buffer_rsrc_t ra_h = make_rsrc(ah, (uint32_t)(kdim * 2u) * a_rows);
     const __amdgpu_buffer_rsrc_t ra_l = make_rsrc(al, (uint32_t)(kdim * 2u) * a_rows);
     const __amdgpu_buffer_rsrc_t rgs = make_rsrc(gs, ngroups * 4u * a_rows);
-    if constexpr (!Q4K && !Q6K) stage_f16_tables<KIND>();
+    if constexpr (!Q4K && !Q6K && !Q8) stage_f16_tables<KIND>();
 
     auto run = [&](auto packed_tag) {
         const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, ln = lane & 15u;
@@ -82,6 +89,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
                 const float2 st = ld_xstat(xstat, pairs ? pairs[q] / K : q);
                 s_rowe[tid] = make_int2(x_exp(st.x), act_exp(st));
             }
+        } else if constexpr (Q8) {
+            if (tid < TMS) s_rowe[tid].x = x_exp(__uint_as_float(rowmax[q0 + (tid < n ? tid : 0u)]));
         } else {
             if (rowmax != nullptr && row0 == 0u) {
                 bool bad = false;
@@ -94,61 +103,52 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
         }
         constexpr bool PK = decltype(packed_tag)::value;
         constexpr uint32_t CH = PK ? 512u : 256u;  // columns per A chunk
-        constexpr uint32_t CS = CH / 64u;          // slabs per chunk
-        constexpr uint32_t ROWT = PK ? 8u : 16u;   // tile rows of the operand
-        constexpr uint32_t DEPTH = 4u;
-        // A staging: item i = tid + 256 j is the 16-byte piece i % (CH / 8) of
-        // operand row i / (CH / 8); items j = 0, 1 are hi rows, j = 2, 3 lo rows.
-        // Piece c of row r sits at slot c ^ (r & 15), so a fragment read (16 rows
-        // at one piece) touches every bank once.
-        const uint32_t ac = tid % (CH / 8u), ar = tid / (CH / 8u);  // + ROWT / 2 rows at odd j
+        constexpr uint32_t CSB = CH / 256u, ROWT = PK ? 8u : 16u, DEPTH = 4u;
+        // A staging: thread tid copies the 16-byte piece tid % (CH / 8) of tile rows
+        // tid / (CH / 8) and ROWT / 2 further, hi and lo (rows past n: an offset past
+        // the buffer, which reads zero without a fetch; no branch, so that the waits
+        // count loads exactly and never drain the B ring).
+        // Operand rows: hi 0 .. ROWT - 1, lo from ROWT; piece c of row r sits at slot
+        // c ^ (r & 15), so a fragment read (16 rows at one piece) touches every bank
+        // once.
+        const uint32_t ac = tid % (CH / 8u), ar = tid / (CH / 8u);
         uint32_t avo[2];
-        bool alive[2];
 #pragma unroll
-        for (uint32_t j = 0; j < 2; ++j) {
-            const uint32_t r = ar + (ROWT / 2u) * j;
-            alive[j] = r < n;
-            const uint32_t q = q0 + (alive[j] ? r : 0u);
-            const uint32_t arow = GATEUP ? (pairs ? pairs[q] / K : q) : q;
-            avo[j] = 2u * (arow * kdim + 8u * ac);
+        for (uint32_t j = 0; j < 2u; ++j) {
+            const uint32_t r = ar + (ROWT / 2u) * j, q = q0 + (r < n ? r : 0u);
+            avo[j] = r < n ? 2u * ((GATEUP && pairs ? pairs[q] / K : q) * kdim + 8u * ac) : 0xffffff00u;
         }
         uint4 areg[4];
         auto load_a = [&](uint32_t c) {
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j)
-                if (alive[j & 1u]) areg[j] = buf_load16(j < 2u ? ra_h : ra_l, avo[j & 1u], 2u * CH * c);
+            for (uint32_t j = 0; j < 4u; ++j) areg[j] = buf_load16(j < 2u ? ra_h : ra_l, avo[j & 1u], 2u * CH * c);
         };
-        auto store_a = [&](uint32_t buf) {
+        auto store_a = [&](_Float16* A) {
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
+            for (uint32_t j = 0; j < 4u; ++j) {
                 const uint32_t r = ar + (ROWT / 2u) * (j & 1u) + (j < 2u ? 0u : ROWT);
-                if (alive[j & 1u])
-                    *reinterpret_cast<uint4*>(&As[buf][r * CH + 8u * (ac ^ (r & 15u))]) = areg[j];
+                *reinterpret_cast<uint4*>(&A[r * CH + 8u * (ac ^ (r & 15u))]) = areg[j];
             }
         };
         // Q4_K group sums: thread tid < 128 owns one (row, group) of the chunk.
         const uint32_t sg = tid % (CH / 32u), sr = tid / (CH / 32u);
-        const bool slive = Q4K && tid < 128u && sr < n;
         float sreg = 0.f;
         uint32_t svo = 0;
         if constexpr (Q4K) {
-            const uint32_t q = q0 + (slive ? sr : 0u);
-            const uint32_t r = GATEUP ? (pairs ? pairs[q] / K : q) : q;
-            svo = 4u * (r * ngroups + sg);
+            const uint32_t q = q0 + (sr < n ? sr : 0u);
+            svo = 4u * ((GATEUP && pairs ? pairs[q] / K : q) * ngroups + sg);
         }
-        auto load_s = [&](uint32_t c) {
-            if (slive) sreg = __uint_as_float(buf_load4(rgs, svo, 4u * (CH / 32u) * c));
-        };
-        auto store_s = [&](uint32_t buf) {
-            if (slive) {
-                _Float16 h, l;
-                split_f16(sreg * 0.03125f, h, l);  // exact; they reach 2^16 for x and 2^19 for act within range
+        auto load_s = [&](uint32_t c) { sreg = __uint_as_float(buf_load4(rgs, svo, (CH / 8u) * c)); };
+        auto store_s = [&](_Float16* S) {
+            _Float16 h, l;
+            split_f16(sreg * 0.03125f, h, l);  // exact; they reach 2^16 for x and 2^19 for act within range
+            if (tid < 128u) {
                 if constexpr (PK) {
-                    Ss[buf][(sg >> 3) * 128u + sr * 8u + (sg & 7u)] = h;
-                    Ss[buf][(sg >> 3) * 128u + (sr + 8u) * 8u + (sg & 7u)] = l;
+                    S[(sg >> 3) * 128u + sr * 8u + (sg & 7u)] = h;
+                    S[(sg >> 3) * 128u + (sr + 8u) * 8u + (sg & 7u)] = l;
                 } else {
-                    Ss[buf][sr * 16u + sg] = h;
-                    Ss[buf][sr * 16u + 8u + sg] = l;
+                    S[sr * 16u + sg] = h;
+                    S[sr * 16u + 8u + sg] = l;
                 }
             }
         };
@@ -160,67 +160,68 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
         if constexpr (!IQN) B.load_hdr(0u);
 #pragma unroll
         for (uint32_t d = 0; d < DEPTH; ++d) B.load_slab(d, d, (d & 1u) == 0u);
-        store_a(0u);
-        if constexpr (Q4K) store_s(0u);
+        store_a(As[0]);
+        if constexpr (Q4K) store_s(Ss[0]);
         __syncthreads();  // A chunk 0, the tables and s_rowe
         typename BS::SbState cur;
         if constexpr (!IQN) B.take_hdr(cur, 0u);
-        const uint32_t chunks = (kdim + CH - 1u) / CH;
-        for (uint32_t c = 0; c < chunks; ++c) {
-            const uint32_t buf = c & 1u;
-            const bool more = c + 1u < chunks;
-            if (more) {
-                load_a(c + 1u);
-                if constexpr (Q4K) load_s(c + 1u);
+        const uint32_t nsb = (slabs + 3u) >> 2;
+        // superblock sb, the part-th of its A chunk
+        auto superblock = [&](uint32_t sb, auto part_tag) {
+            constexpr uint32_t PART = decltype(part_tag)::value;
+            const uint32_t c = sb / CSB;
+            const _Float16* const A = As[c & 1u];
+            const bool more = (c + 1u) * CSB < nsb;
+            if constexpr (PART == 0u) {
+                load_a(more ? c + 1u : c);
+                if constexpr (Q4K) load_s(more ? c + 1u : c);
             }
-            const _Float16* const A = As[buf];
+            floatx4 acc[NB];
 #pragma unroll
-            for (uint32_t sbi = 0; sbi < CS / 4u; ++sbi) {
-                const uint32_t sb = c * (CS / 4u) + sbi;
-                if (4u * sb >= slabs) break;  // uniform
-                floatx4 acc[NB];
+            for (int nb = 0; nb < NB; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) acc[nb] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (uint32_t sq = 0; sq < 4u; ++sq) {
+                const uint32_t s = 4u * sb + sq;
+                // B of slab s out of the ring, B(s + DEPTH) into its slot
+                uint4 qv[NB];
+                uint32_t ex[NB];
+                uint2 dv[NB];
 #pragma unroll
-                for (uint32_t sq = 0; sq < 4u; ++sq) {
-                    const uint32_t s = 4u * sb + sq;
-                    if constexpr (IQN) {
-                        if (s >= slabs) break;  // uniform
-                    }
-                    // B of slab s out of the ring, B(s + DEPTH) into its slot
-                    uint4 qv[NB];
-                    uint2 dv[NB];
+                for (int nb = 0; nb < NB; ++nb) {
+                    qv[nb] = B.nq[sq][nb];
+                    if constexpr (IQN && !Q8) qv[nb].z = B.n1[sq][nb];
+                    if constexpr (Q8) ex[nb] = B.n1[sq][nb];
+                    if constexpr (IQN || Q6K) dv[nb] = B.nd[sq][nb];
+                }
+                half8 fb[NB][2], fe[NB][2];
+                float dg[NB][2];
+                B.decode(cur, sq, qv, dv, fb, dg, fe, ex);
+                B.load_slab(sq, s + DEPTH, (sq & 1u) == 0u);
+                if constexpr (!IQN) {
+                    if (sq == 0) B.load_hdr(sb + 1u);
+                }
+#pragma unroll
+                for (uint32_t gi = 0; gi < 2; ++gi) {
+                    const uint32_t cn = 32u * PART + 8u * sq + (IQG ? 2u * kq + gi : 4u * gi + kq);
+                    const uint32_t ch = XORD == A_NATURAL ? cn : a_pos<XORD>(8u * cn) >> 3;
+                    const half8 a0 = *reinterpret_cast<const half8*>(&A[ln * CH + 8u * (ch ^ ln)]);
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {
-                        qv[nb] = B.nq[sq][nb];
-                        if constexpr (IQN) qv[nb].z = B.n1[sq][nb];
-                        if constexpr (IQN || Q6K) dv[nb] = B.nd[sq][nb];
+                        const floatx4 z = IQN ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[nb];
+                        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, fb[nb][gi], z, 0, 0, 0);
+                        if constexpr (Q6K)
+                            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, fe[nb][gi], acc[nb], 0, 0, 0);
                     }
-                    half8 fb[NB][2], fe[NB][2];
-                    float dg[NB][2];
-                    B.decode(cur, sq, qv, dv, fb, dg, fe);
-                    B.load_slab(sq, s + DEPTH, (sq & 1u) == 0u);
-                    if constexpr (!IQN) {
-                        if (sq == 0) B.load_hdr(sb + 1u);
+                    if constexpr (!PK) {
+                        const half8 a1 = *reinterpret_cast<const half8*>(&A[(16u + ln) * CH + 8u * (ch ^ ln)]);
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, fb[nb][gi], acc[nb], 0, 0, 0);
                     }
-#pragma unroll
-                    for (uint32_t gi = 0; gi < 2; ++gi) {
-                        const uint32_t ch = 8u * (4u * sbi + sq) + (IQG ? 2u * kq + gi : 4u * gi + kq);
-                        const half8 a0 = *reinterpret_cast<const half8*>(&A[ln * CH + 8u * (ch ^ ln)]);
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            const floatx4 z = IQN ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[nb];
-                            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, fb[nb][gi], z, 0, 0, 0);
-                            if constexpr (Q6K)
-                                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, fe[nb][gi], acc[nb], 0, 0, 0);
-                        }
-                        if constexpr (!PK) {
-                            const half8 a1 = *reinterpret_cast<const half8*>(&A[(16u + ln) * CH + 8u * (ch ^ ln)]);
-#pragma unroll
-                            for (int nb = 0; nb < NB; ++nb)
-                                acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, fb[nb][gi], acc[nb], 0, 0, 0);
-                        }
-                        if constexpr (IQN) {
+                    if constexpr (IQN) {
+                        // (a last superblock cut short: clamped weights over columns past K,
+                        // not added)
+                        if (s < slabs) {
 #pragma unroll
                             for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
@@ -228,34 +229,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
                         }
                     }
                 }
-                if constexpr (!IQN) {
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) tot[nb][j] += cur.dsc[nb] * acc[nb][j];
-                    if constexpr (Q4K) {
-                        const half8 sa = *reinterpret_cast<const half8*>(
-                            PK ? &Ss[buf][sbi * 128u + ln * 8u] : &Ss[buf][ln * 16u + 8u * (kq & 1u)]);
-#pragma unroll
-                        for (int nb = 0; nb < NB; ++nb) {
-                            const uint4 v = kq < (PK ? 1u : 2u)
-                                                ? make_uint4(bytes01(cur.mn[nb][0]), bytes23(cur.mn[nb][0]),
-                                                             bytes01(cur.mn[nb][1]), bytes23(cur.mn[nb][1]))
-                                                : make_uint4(0, 0, 0, 0);
-                            const floatx4 mc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                sa, __builtin_bit_cast(half8, v), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) tot[nb][j] -= cur.dmn[nb] * mc[j];
-                        }
-                    }
-                    B.take_hdr(cur, sb + 1u);  // past the last superblock: the clamped header, never used
-                }
             }
-            if (more) {
-                // the other buffer was last read in chunk c - 1, before the last barrier
-                store_a(buf ^ 1u);
-                if constexpr (Q4K) store_s(buf ^ 1u);
+            if constexpr (!IQN) {
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) tot[nb][j] += cur.dsc[nb] * acc[nb][j];
+                if constexpr (Q4K) {
+                    const half8 sa = *reinterpret_cast<const half8*>(
+                        &Ss[c & 1u][PK ? PART * 128u + ln * 8u : ln * 16u + 8u * (kq & 1u)]);
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) {
+                        const uint4 v = kq < (PK ? 1u : 2u) ? make_uint4(bytes01(cur.mn[nb][0]), bytes23(cur.mn[nb][0]),
+                                                                         bytes01(cur.mn[nb][1]), bytes23(cur.mn[nb][1]))
+                                                            : make_uint4(0, 0, 0, 0);
+                        const floatx4 mc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            sa, __builtin_bit_cast(half8, v), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) tot[nb][j] -= cur.dmn[nb] * mc[j];
+                    }
+                }
+                B.take_hdr(cur, sb + 1u);  // past the last superblock: the clamped header, never used
+            }
+            if (PART + 1u == CSB && more) {
+                // the other buffer was last read before the last barrier
+                store_a(As[(c + 1u) & 1u]);
+                if constexpr (Q4K) store_s(Ss[(c + 1u) & 1u]);
                 __syncthreads();
+            }
+        };
+        for (uint32_t sb = 0; sb < nsb; sb += CSB) {
+            superblock(sb, std::integral_constant<uint32_t, 0>{});
+            if constexpr (CSB == 2u) {
+                if (sb + 1u >= nsb) break;
+                superblock(sb + 1u, std::integral_constant<uint32_t, 1>{});
             }
         }
         // packed: rows 8..15 hold the lo products of rows 0..7 (lane + 32)
@@ -275,15 +282,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
             if constexpr (GATEUP) {
                 // g, u in true units, then act 2^a_t; act column row0 + 16 w + ln
                 const int ex = s_rowe[m].x, ea = s_rowe[m].y;
-                const float v = ldexpf(swiglu(ldexpf(tot[0][j], -ex), ldexpf(tot[1][j], -ex), limit), ea);
-                // the row's max |act| over the 16 lanes of this row (bit patterns as
-                // integers: NaN stays above infinity)
-                uint32_t rm = __float_as_uint(fabsf(v));
-                rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0xb1, 0xf, 0xf, false));
-                rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x4e, 0xf, 0xf, false));
-                rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x141, 0xf, 0xf, false));
-                rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x140, 0xf, 0xf, false));
+                const float sw = swiglu(ldexpf(tot[0][j], -ex), ldexpf(tot[1][j], -ex), limit);
+                const float v = Q8 ? sw : ldexpf(sw, ea);
+                const uint32_t rm = row_max16(__float_as_uint(fabsf(v)));
                 if (own && ln == 0u) rpart[wave][m] = rm;
+                if constexpr (Q8) {
+                    if (live) out[q * ldo + row0 + 16u * wave + ln] = v;
+                    continue;
+                }
                 _Float16 hh, ll;
                 split_f16(v, hh, ll);
                 if (live) {
@@ -302,7 +308,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
             } else if (live) {
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb)
-                    out[q * ldo + row0 + 32u * wave + 16u * nb + ln] = tot[nb][j];
+                    out[q * ldo + row0 + 32u * wave + 16u * nb + ln] = Q8 ? ldexpf(tot[nb][j], -s_rowe[m].x) : tot[nb][j];
             }
         }
         if constexpr (GATEUP) {

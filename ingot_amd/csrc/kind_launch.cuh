@@ -161,7 +161,9 @@ bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, 
     } while (0)
 #define F16A(TT)                                  \
     do {                                          \
-        if constexpr (GATEUP) {                   \
+        if constexpr (GATEUP && KIND == 8) {      \
+            F16T(A_F32, TT);                      \
+        } else if constexpr (GATEUP) {            \
             switch (aord) {                       \
                 case A_IQ4NL: F16T(A_IQ4NL, TT);  \
                 case A_IQ3XXS: F16T(A_IQ3XXS, TT); \
@@ -186,8 +188,8 @@ bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, 
 
 template <int KIND, bool GATEUP>
 void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a) {
-#define SML_(AO, TLV)                                                                                            \
-    hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
+#define SML_(AO, TLV, ...)                                                                                       \
+    hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV, ##__VA_ARGS__>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
                        a.e_shared, a.stride0, a.stride1, a.rows_per_expert, a.kdim, a.ah, a.al, a.gs, a.pairs,   \
                        a.K, a.tiles, a.ldo, a.limit, a.out, a.out_h, a.out_l, a.out_gs, a.nblk, a.a_rows,        \
                        a.xstat, a.rowmax, a.flags, a.slot_of)
@@ -197,7 +199,13 @@ void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const Gemm
         else SML_(AO, false);   \
         return;                 \
     } while (0)
-    if constexpr (GATEUP) {
+    if constexpr (GATEUP && KIND == 8) {
+        // act in fp32; aord is the order in which x is stored (a dense product reads
+        // GGUF order, the routed experts' x is natural)
+        if (aord == A_IQ3XXS) SML_(A_F32, false, A_IQ3XXS);
+        else if (aord == A_Q6K) SML_(A_F32, false, A_Q6K);
+        else SML(A_F32);
+    } else if constexpr (GATEUP) {
         switch (aord) {
             case A_IQ4NL: SML(A_IQ4NL);
             case A_IQ3XXS: SML(A_IQ3XXS);

@@ -132,12 +132,13 @@ struct GemmF16Args {
     const uint32_t* slot_of;
 };
 // The formats of the f16 grouped GEMM.
-#define INGOT_F16_KINDS(X) X(12) X(13) X(14) X(17) X(18) X(20) X(21) X(22) X(23)
+#define INGOT_F16_KINDS(X) X(8) X(12) X(13) X(14) X(17) X(18) X(20) X(21) X(22) X(23)
 // k_gemm_f16<KIND, GATEUP, aord, TT, tl>: TT 128 when tt128 (Q4_K, Q5_K; Q6_K
 // always), else 64; false if no instantiation covers the arguments.
 template <int KIND, bool GATEUP>
 bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, const GemmF16Args& a);
-// k_gemm_small<KIND, GATEUP, aord, tl>: the same over tiles of at most TMS pairs.
+// k_gemm_small<KIND, GATEUP, aord, tl>: the same over tiles of at most TMS pairs
+// (Q8_0 gate/up: aord is the column order of x).
 template <int KIND, bool GATEUP>
 void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a);
 

@@ -199,7 +199,7 @@ bool tiled_kind(const DevMatrix& m) {
     switch (m.kind) {
         case 12: case 13: case 14: case 23: cols_ok = m.cols % 256 == 0; break;
         case 17: case 18: case 21: case 22: cols_ok = m.cols % 512 == 0; break;
-        case 20: cols_ok = m.cols % 64 == 0; break;
+        case 8: case 20: cols_ok = m.cols % 64 == 0; break;
         default: break;
     }
     return cols_ok && m.rows % 16 == 0;
@@ -358,7 +358,7 @@ bool f16_gemm_kind(uint32_t kind, uint32_t kdim, bool gateup) {
         case 12: case 13: return kdim % 256 == 0;
         case 14: return kdim % 256 == 0;
         case 17: case 18: case 21: case 22: return kdim % 512 == 0;
-        case 20: return kdim % 64 == 0;
+        case 8: case 20: return kdim % 64 == 0;
         case 23: return kdim % 256 == 0;
         default: return false;
     }
@@ -718,18 +718,27 @@ static bool f16_gemm_fits(uint64_t kdim, uint64_t rows) { return 2ull * kdim * r
 // fp32 act for the fp32 down GEMM); f16: down too; merge: the shared expert
 // joins the same launches (its formats and width equal the routed experts').
 struct PrefillPlan {
-    bool f16gu = false, f16 = false, merge = false;
+    bool f16gu = false, f16 = false, merge = false, dense8 = false;
 };
 
 static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
     PrefillPlan p;
     const uint64_t P = (uint64_t)T * L->K, PS = P + (L->has_shared ? T : 0u);
+    // Q8_0 on both projections or neither: its gate/up hands act over in fp32 with
+    // its row maxima (k_split_act), the other formats' in units of the token.
+    const bool q8 = L->gate.kind == 8;
     p.f16gu = L->gemm_mode == INGOT_GEMM_AUTO && f16_gemm_kind(L->gate.kind, L->H, true) && f16_gemm_fits(L->H, T) &&
-              f16_gemm_fits(L->F, PS);
-    p.f16 = p.f16gu && f16_gemm_kind(L->down.kind, L->F, false);
+              f16_gemm_fits(L->F, PS) && (!q8 || L->down.kind == 8);
+    p.f16 = p.f16gu && f16_gemm_kind(L->down.kind, L->F, false) && (q8 || L->down.kind != 8);
     p.merge = p.f16 && L->has_shared && L->SF == L->F && L->sgate.kind == L->gate.kind &&
               L->sup.kind == L->up.kind && L->sdown.kind == L->down.kind && L->sgate.stride == L->gate.stride &&
               L->sup.stride == L->up.stride && L->sdown.stride == L->down.stride;
+    // A Q8_0 shared expert that does not join: k_gemm_small over dense tiles, where
+    // x is stored in an order it can look up; rows P .. of acth / actl hold its act.
+    // (512 experts, IQ2_XS, at 509 tokens: 64 + 128 blocks of the fp32 GEMM took 55
+    // and 14 us.)
+    p.dense8 = p.f16gu && L->has_shared && !p.merge && L->sgate.kind == 8 && L->sdown.kind == 8 && L->SF <= L->F &&
+               a_order(L->gate.kind) != A_IQ4NL;
     return p;
 }
 
@@ -1556,8 +1565,9 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         // f16 GEMM writing fp32 act and the down projection on the fp32 GEMM,
         // over the same 64-token tiles.
         const PrefillPlan plan = prefill_plan(L, T);
-        const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge;
-        const int aord = f16 ? a_order(down.kind) : A_F32, xord = a_order(gate.kind);
+        const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge, dense8 = plan.dense8;
+        const bool q8 = f16 && gate.kind == 8;
+        const int xord = a_order(gate.kind), aord = q8 ? xord : f16 ? a_order(down.kind) : A_F32;
         const bool mins = f16 && (down.kind == 12 || down.kind == 13);
         // 128-token tiles when an expert can take more than 64 pairs (each takes at
         // most one per token), the launch averages at least 32 pairs per expert
@@ -1574,10 +1584,11 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         const bool tlg = f16gu && gate.t && up.t && (!merge || (sgate.t && sup.t));
         const bool tld = f16 && down.t && (!merge || sdown.t);
         // The small-tile GEMM up to SMALL_PAIRS_PER_EXPERT pairs per expert on average;
-        // its tile list lies in w.act, which only an fp32 down GEMM uses.
+        // its tile list lies in w.act, which only an fp32 down GEMM and Q8_0 use (Q8_0:
+        // in w.acts, the group sums that only Q4_K and Q5_K use).
         const uint32_t pcap = (P + TMS - 1) / TMS + E + (merge ? (T + TMS - 1) / TMS : 0u);
-        const bool small = f16 && P <= SMALL_PAIRS_PER_EXPERT * E && 16ull * pcap <= 4ull * P * F;
-        uint32_t* const ptiles = small ? reinterpret_cast<uint32_t*>(w.act) : nullptr;
+        const bool small = f16 && P <= SMALL_PAIRS_PER_EXPERT * E && 16ull * pcap <= (q8 ? 4ull * P * (F / 32) : 4ull * P * F);
+        uint32_t* const ptiles = small ? reinterpret_cast<uint32_t*>(q8 ? w.acts : w.act) : nullptr;
         const uint32_t tm = tt128 ? 2u * TM : TM;
         const uint8_t *g16 = tlg ? gate.t : gate.d, *u16 = tlg ? up.t : up.d, *d16 = tld ? down.t : down.d;
         const uint8_t *sg16 = tlg ? sgate.t : sgate.d, *su16 = tlg ? sup.t : sup.d, *sd16 = tld ? sdown.t : sdown.d;
@@ -1585,13 +1596,19 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         _Float16 *xh = w.xh, *xl = w.xl, *acth = w.acth, *actl = w.actl;
         float *xs = w.xs, *acts = w.acts;
         // rows whose maxima the f16 gate/up raises (act split in the f16 GEMM's units)
-        uint32_t* rmx = f16 ? rowmax : nullptr;
-        const uint32_t nrow = f16 ? P + S : 0u;
+        uint32_t *rmx = f16 ? rowmax : nullptr, *rmz = f16 || dense8 ? rowmax : nullptr;
+        const uint32_t nrow = rmz ? P + (merge || dense8 ? T : 0u) : 0u;
         L->last_T = T;
         L->last_P = P;
         L->last_S = S;
         L->last_cap = capf;
         L->last_tm = tm;
+        auto split_act = [](hipStream_t ss, const float* a, const uint32_t* rm, uint64_t rows, uint32_t f, _Float16* h,
+                            _Float16* l) {
+            const uint64_t n = rows * f;
+            hipLaunchKernelGGL(k_split_act, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, ss, a, rm, n, f, h, l);
+        };
+        auto dense_grid = [T](uint32_t nblk) { return dim3(8 * nblk * (((T + TMS - 1) / TMS + 7) / 8)); };
         // Dispatch stage: expert grouping, and for the f16 GEMM the split of x
         // into f16 hi/lo with its 32-column sums.
         L->stage[ST_DISPATCH] = [=](hipStream_t ss) {
@@ -1599,9 +1616,9 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             const uint64_t n = f16gu ? (uint64_t)T * H : 0ull;
             const uint32_t nsplit = (uint32_t)((n / 4 + 1023) / 1024);
             hipLaunchKernelGGL(k_dispatch, dim3(1 + nsplit), dim3(1024), 0, ss, ids, P, E, tm, capf, counts, first, tiles,
-                               pairs, inverse, S, K, xin, n, xh, xl, xs, (uint32_t)xord, (const float*)xstat, H, rmx,
+                               pairs, inverse, S, K, xin, n, xh, xl, xs, (uint32_t)xord, (const float*)xstat, H, rmz,
                                nrow, ptiles, pcap);
-            if (hs && !merge)
+            if (hs && !merge && !dense8)
                 hipLaunchKernelGGL(k_dense_tiles, dim3((scap + 63) / 64), dim3(64), 0, ss, T, scap, stiles);
         };
         L->stage_name[ST_DISPATCH] = "k_dispatch";
@@ -1612,7 +1629,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                 launch_gemm_small<true>(ss, gate.kind, aord, tlg, dim3(8 * (F / 64) * ((pcap + 7) / 8)), g16, u16,
                                         merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride, F,
                                         H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
-                                        (const uint32_t*)pairs, K, (const uint32_t*)ptiles, F, limit, (float*)nullptr,
+                                        (const uint32_t*)pairs, K, (const uint32_t*)ptiles, F, limit, q8 ? act : (float*)nullptr,
                                         acth, actl, mins ? acts : nullptr, F / 64, T, (const float*)xstat, rmx, flags,
                                         so);
             } else if (f16gu) {
@@ -1620,13 +1637,22 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                       merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride,
                                       F, H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
                                       (const uint32_t*)pairs, K, (const uint32_t*)tiles, F, limit,
-                                      f16 ? (float*)nullptr : act, acth, actl, mins ? acts : nullptr, F / 64, T,
+                                      f16 && !q8 ? (float*)nullptr : act, acth, actl, mins ? acts : nullptr, F / 64, T,
                                       (const float*)xstat, rmx, flags, so);
             } else {
                 launch_gemm<true>(ss, gate.kind, dim3(F / 64, cap), gate.d, up.d, gate.stride, up.stride, F, H, xin,
                                   pairs, K, tiles, F, limit, act, so);
             }
-            if (hs && !merge && LL->pass.first)
+            if (q8) split_act(ss, act, rmx, (uint64_t)(P + S), F, acth, actl);
+            if (dense8 && LL->pass.first) {
+                launch_gemm_small<true>(ss, 8u, xord, false, dense_grid(SF / 64), (const uint8_t*)sgate.d,
+                                        (const uint8_t*)sup.d, (const uint8_t*)nullptr, (const uint8_t*)nullptr,
+                                        0xffffffffu, sgate.stride, sup.stride, SF, H, (const _Float16*)xh,
+                                        (const _Float16*)xl, (const float*)nullptr, (const uint32_t*)nullptr, 1u,
+                                        (const uint32_t*)nullptr, SF, limit, sact, (_Float16*)nullptr,
+                                        (_Float16*)nullptr, (float*)nullptr, SF / 64, T, (const float*)xstat,
+                                        rowmax + P, flags, (const uint32_t*)nullptr);
+            } else if (hs && !merge && LL->pass.first)
                 launch_gemm<true>(ss, sgate.kind, dim3(SF / 64, scap), sgate.d, sup.d, sgate.stride, sup.stride, SF, H,
                                   xin, nullptr, 1, stiles, SF, limit, sact);
         };
@@ -1650,13 +1676,23 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             else
                 launch_gemm<false>(ss, down.kind, dim3(H / 128, cap), down.d, nullptr, down.stride, 0, H, F, act,
                                    nullptr, K, tiles, H, 0.f, Y, so);
-            if (hs && !merge && LL->pass.first)
+            if (dense8 && LL->pass.first) {
+                _Float16 *sh = acth + (uint64_t)P * F, *sl = actl + (uint64_t)P * F;
+                split_act(ss, sact, rowmax + P, T, SF, sh, sl);
+                launch_gemm_small<false>(ss, 8u, A_NATURAL, false, dense_grid(H / 128), (const uint8_t*)sdown.d,
+                                         (const uint8_t*)nullptr, (const uint8_t*)nullptr, (const uint8_t*)nullptr,
+                                         0xffffffffu, sdown.stride, 0ull, H, SF, (const _Float16*)sh,
+                                         (const _Float16*)sl, (const float*)nullptr, (const uint32_t*)nullptr, 1u,
+                                         (const uint32_t*)nullptr, H, 0.f, Ys, (_Float16*)nullptr, (_Float16*)nullptr,
+                                         (float*)nullptr, H / 128, T, (const float*)xstat, rowmax + P, flags,
+                                         (const uint32_t*)nullptr);
+            } else if (hs && !merge && LL->pass.first)
                 launch_gemm<false>(ss, sdown.kind, dim3(H / 128, scap), sdown.d, nullptr, sdown.stride, 0, H, SF, sact,
                                    nullptr, 1, stiles, H, 0.f, Ys);
         };
         L->stage_name[ST_DOWN] = f16 ? "k_gemm_f16<down>" : "k_gemm<down>";
-        // The f16 down GEMM's rows of Y are in the act units of their token.
-        const float* yscale = f16 ? xstat : nullptr;
+        // The f16 down GEMM's rows of Y are in the act units of their token (Q8_0: true units).
+        const float* yscale = f16 && !q8 ? xstat : nullptr;
         const uint32_t shared_scaled = merge ? 1u : 0u;
         L->stage[ST_COMBINE] = [=](hipStream_t ss) {
             hipLaunchKernelGGL(k_combine, dim3((H / 4 + 255) / 256, T), dim3(256), 0, ss, Y, hs ? Ys : nullptr,

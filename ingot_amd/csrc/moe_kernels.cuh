@@ -2079,12 +2079,17 @@ constexpr uint32_t TILE_Q4K = 2304, TILE_IQ3XXS = 1568, TILE_IQ4NL = 576;
 //     the row's 16 scale bytes; at 3328 + 2 ln its d.
 constexpr uint32_t TILE_Q5K = 2816, TILE_IQ2XS = 1184, TILE_IQ2S = 1312, TILE_IQ3S = 1760, TILE_IQ4XS = 2176,
                    TILE_Q6K = 3360;
+//   Q8_0 (1088 per slab of two 34-byte blocks): at 16 l the bytes
+//     2 + 8 kq .. + 7 of the slab's first block, then those of its second; at
+//     1024 + 4 ln the row's two d.
+constexpr uint32_t TILE_Q80 = 1088;
 __host__ __device__ constexpr uint32_t tile_record(int kind) {
     return kind == 12   ? TILE_Q4K
            : kind == 13 ? TILE_Q5K
            : kind == 14 ? TILE_Q6K
            : kind == 17 ? TILE_IQ2XS
            : kind == 18 ? TILE_IQ3XXS
+           : kind == 8  ? TILE_Q80
            : kind == 20 ? TILE_IQ4NL
            : kind == 21 ? TILE_IQ3S
            : kind == 22 ? TILE_IQ2S
@@ -2107,6 +2112,15 @@ __device__ __forceinline__ uint2 buf_load8(__amdgpu_buffer_rsrc_t r, uint32_t vo
 }
 __device__ __forceinline__ uint32_t buf_load4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
     return __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0);
+}
+
+// The maximum over the 16 lanes of a row (bit patterns of |v| as integers: NaN
+// stays above infinity).
+__device__ __forceinline__ uint32_t row_max16(uint32_t rm) {
+    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0xb1, 0xf, 0xf, false));
+    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x4e, 0xf, 0xf, false));
+    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x141, 0xf, 0xf, false));
+    return max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x140, 0xf, 0xf, false));
 }
 
 // s_waitcnt vmcnt(N) alone (expcnt and lgkmcnt fields at their maxima).
@@ -2150,7 +2164,10 @@ struct BStream {
     // block): its blocks' 16 quant bytes sit at 8 + 16 g of a 136-byte
     // superblock (dword aligned), and a block's unit is d * (scale - 32), the
     // 6-bit scale from the 8-byte superblock header read with each slab.
-    static constexpr bool IQ4X = KIND == 23, IQN = IQ4 || IQ4X;
+    static constexpr bool IQ4X = KIND == 23;
+    // Q8_0 too (34-byte blocks): B the int8 value as an f16 integer (no 2^-24
+    // unit), a block's unit its d.
+    static constexpr bool Q8 = KIND == 8, IQN = IQ4 || IQ4X || Q8;
     // Q6_K (210-byte superblocks, kernels/moe.metal:22-28): w = d sc (q - 32),
     // q = 4 bits of ql | 2 bits of qh, sc an int8 per 16 columns; |sc (q - 32)|
     // reaches 4096, past the 2048 that f16 holds exactly, so B enters twice:
@@ -2318,6 +2335,18 @@ struct BStream {
                 n1[rs][nb] = q.y;
                 const uint32_t dw = buf_load4(rw, 4u * ln, u + 512u);
                 nd[rs][nb] = make_uint2(dw, dw);
+            } else if constexpr (TL && Q8) {
+                const uint32_t u = bsoff[nb] + TREC * s;
+                nq[rs][nb] = buf_load16(rw, 16u * lane, u);
+                nd[rs][nb].x = buf_load4(rw, 4u * ln, u + 1024u);
+            } else if constexpr (Q8) {
+                // the first block's bytes 2 bytes off a dword, the second's on one
+                const uint32_t u = bsoff[nb] + 68u * s;
+                const auto a = __builtin_amdgcn_raw_buffer_load_b96(rw, (int)(boff[nb] + 8u * kq), (int)u, 0);
+                const uint2 b = buf_load8(rw, boff[nb] + 8u * kq, u + 36u);
+                nq[rs][nb] = make_uint4(a[0], a[1], b.x, b.y);
+                n1[rs][nb] = a[2];
+                nd[rs][nb] = make_uint2(buf_load4(rw, boff[nb], u), buf_load4(rw, boff[nb], u + 32u));
             } else if constexpr (IQ4) {
                 const uint32_t u = bsoff[nb] + 36u * s;
                 const uint2 q = buf_load8(rw, boff[nb] + 4u * kq, u);
@@ -2447,7 +2476,8 @@ struct BStream {
     // into fb, B_e into fe); IQ4_NL also yields the units of its two blocks and
     // whether a d is zero.
     __device__ __forceinline__ void decode(const SbState& st, uint32_t sq, const uint4* qv, const uint2* dv,
-                                           half8 (*fb)[2], float (*dg)[2], half8 (*fe)[2]) {
+                                           half8 (*fb)[2], float (*dg)[2], half8 (*fe)[2],
+                                           const uint32_t* ex = nullptr) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             if constexpr (Q6K) {
@@ -2567,6 +2597,29 @@ struct BStream {
                         half8, make_uint4(mad_u16x2(e0.x, f2, m.x), mad_u16x2(e0.y, f2, m.y),
                                           mad_u16x2(e1.x, f2, m.z), mad_u16x2(e1.y, f2, m.w)));
                 }
+            } else if constexpr (Q8) {
+                // int8 q -> f16 bits 0x6400 | (q ^ 0x80) = 1152 + q, minus 1152
+                const float d[2] = {half_bits_to_float(dv[nb].x & 0xffffu),
+                                    half_bits_to_float((TL ? dv[nb].x : dv[nb].y) >> 16)};
+                // (GGUF order: the first block's bytes from their window, its third word in ex)
+                const uint32_t w[4] = {TL ? qv[nb].x : __builtin_amdgcn_alignbit(qv[nb].y, qv[nb].x, 16u),
+                                       TL ? qv[nb].y : __builtin_amdgcn_alignbit(ex[nb], qv[nb].y, 16u), qv[nb].z,
+                                       qv[nb].w};
+#pragma unroll
+                for (int gi = 0; gi < 2; ++gi) {
+                    uint32_t b[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t u = __builtin_amdgcn_perm(0x64646464u, w[2 * gi + (i >> 1)] ^ 0x80808080u,
+                                                                 (i & 1) ? 0x04030402u : 0x04010400u);
+                        b[i] = __builtin_bit_cast(
+                            uint32_t, __builtin_bit_cast(half2v, u) - half2v{(_Float16)1152.f, (_Float16)1152.f});
+                    }
+                    // (a zero d zeroes B: the unit is then 1)
+                    fb[nb][gi] = __builtin_bit_cast(half8, d[gi] != 0.f ? make_uint4(b[0], b[1], b[2], b[3])
+                                                                        : make_uint4(0u, 0u, 0u, 0u));
+                    dg[nb][gi] = d[gi] != 0.f ? d[gi] : 1.f;
+                }
             } else {
                 uint32_t qa, qb;
                 float d0, d1;
@@ -2656,9 +2709,9 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     float* __restrict__ out, _Float16* __restrict__ out_h, _Float16* __restrict__ out_l, float* __restrict__ out_gs,
     uint32_t nblk, uint32_t a_rows, const float* __restrict__ xstat, uint32_t* __restrict__ rowmax,
     uint32_t* __restrict__ flags, const uint32_t* __restrict__ slot_of) {
-    static_assert(KIND == 12 || KIND == 13 || KIND == 14 || KIND == 17 || KIND == 18 || KIND == 20 || KIND == 21 ||
+    static_assert(KIND == 8 || KIND == 12 || KIND == 13 || KIND == 14 || KIND == 17 || KIND == 18 || KIND == 20 || KIND == 21 ||
                       KIND == 22 || KIND == 23,
-                  "f16 GEMM formats: Q4_K, Q5_K, Q6_K, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_NL, IQ4_XS");
+                  "f16 GEMM formats: Q8_0, Q4_K, Q5_K, Q6_K, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_NL, IQ4_XS");
     static_assert(AORD == A_NATURAL || GATEUP, "the permuted act layout is written by the gate/up kernel");
     static_assert(TT == 64 || TT == 128, "tiles of 64 or 128 tokens");
     // NB: 16-row B blocks per wave (gate/up: HB = NB / 2 gate, HB up); NW waves.
@@ -2666,7 +2719,11 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     constexpr uint32_t NW = TT / 32u, HB = NB / 2;
     using BS = BStream<KIND, NB, GATEUP, TL>;
     constexpr bool Q5K = BS::Q5K, Q4K = BS::Q4K, IQ2S = BS::IQ2S, IQ3S = BS::IQ3S, IQG = BS::IQG, IQ4 = BS::IQ4,
-                   IQ4X = BS::IQ4X, IQN = BS::IQN, Q6K = BS::Q6K;
+                   IQ4X = BS::IQ4X, IQN = BS::IQN, Q6K = BS::Q6K, Q8 = BS::Q8;
+    // Q8_0 layers: gate/up writes act in fp32 with its row maxima, k_split_act
+    // splits it by them, and the down product returns to true units here, so no
+    // activation leaves the f16 range.
+    static_assert(!Q8 || !GATEUP || AORD == A_F32, "Q8_0 gate/up writes fp32 act");
     // (two operand sets per fragment: TT 128's 2 row blocks per wave fit the registers, 4 do not)
     static_assert(!Q6K || TT == 128, "Q6_K runs on 128-token tiles (which also take tiles of 64)");
     constexpr uint32_t UNR = 4u;
@@ -2695,7 +2752,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     // pass (NO_SLOT) and the tile waits for a later one.
     const uint32_t ew = slot_of ? slot_of[tile[0]] : tile[0];
     if (ew == NO_SLOT) return;
-    if constexpr (!Q4K && !Q6K) {
+    if constexpr (!Q4K && !Q6K && !Q8) {
         stage_f16_tables<KIND>();
         __syncthreads();
     }
@@ -2741,6 +2798,8 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
             const float2 st = ld_xstat(xstat, pairs ? pairs[q] / K : q);
             s_rowe[tid] = make_int2(x_exp(st.x), act_exp(st));
         }
+    } else if constexpr (Q8) {
+        if (tid < TT) s_rowe[tid].x = x_exp(__uint_as_float(rowmax[q0 + (tid < n ? tid : 0u)]));
     } else {
         if (rowmax != nullptr && slot - ti * nblk == 0u) {
             bool bad = false;
@@ -2775,7 +2834,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     };
     // Vector-memory loads issued after a slab's A DMA: the B ring's, and at a
     // superblock's first slab its header (and Q4_K group sums).
-    constexpr uint32_t B_PER_SLAB = Q4K ? NB : IQ4 ? (TL ? 2u : 4u) * NB : IQ4X ? (TL ? 2u : 3u) * NB : 0u;
+    constexpr uint32_t B_PER_SLAB = Q4K ? NB : IQ4 || Q8 ? (TL ? 2u : 4u) * NB : IQ4X ? (TL ? 2u : 3u) * NB : 0u;
     constexpr uint32_t B_PER_SB = Q5K                ? 2u * NB + 1u
                                   : Q4K              ? NB + 1u
                                   : IQ2S             ? (TL ? 3u : 7u) * NB
@@ -2826,15 +2885,17 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
         float dgs[NFB][NB][2];
         {
             uint4 qv[NB];
+            uint32_t ex[NB];
             uint2 dv[NB];
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 qv[nb] = B.nq[0][nb];
-                if constexpr (IQN) qv[nb].z = B.n1[0][nb];
+                if constexpr (IQN && !Q8) qv[nb].z = B.n1[0][nb];
+                if constexpr (Q8) ex[nb] = B.n1[0][nb];
                 if constexpr (IQN || Q6K) dv[nb] = B.nd[0][nb];
             }
             B.load_slab(0, DEPTH, true);
-            B.decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0]);
+            B.decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0], ex);
         }
         for (uint32_t s0 = 0; s0 < slabs; s0 += UNR) {
             const uint32_t sb = s0 >> 2;
@@ -2857,11 +2918,13 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 // B of slab s + 1 out of the ring, B(s + 1 + DEPTH) into its slot.
                 const uint32_t rs = (sq + 1u) % DEPTH;
                 uint4 qv[NB];
+                uint32_t ex[NB];
                 uint2 dv[NB];
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     qv[nb] = B.nq[rs][nb];
-                    if constexpr (IQN) qv[nb].z = B.n1[rs][nb];
+                    if constexpr (IQN && !Q8) qv[nb].z = B.n1[rs][nb];
+                    if constexpr (Q8) ex[nb] = B.n1[rs][nb];
                     if constexpr (IQN || Q6K) dv[nb] = B.nd[rs][nb];
                 }
                 // (s is a multiple of UNR plus sq: slab s + 1 + DEPTH opens a half when sq is odd)
@@ -2881,7 +2944,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 const uint32_t cb = NFB == 2u ? (sq & 1u) : 0u, nb_ = NFB == 2u ? cb ^ 1u : 0u;
                 // (after the last slab: a decode of clamped bytes that nothing reads;
                 // kept unconditional so that the decode shares a block with the MFMAs)
-                if (NFB == 2u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u]);
+                if (NFB == 2u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u], ex);
                 const _Float16* const bh = (sq & 1u) ? Ah1 : Ah0;
                 const _Float16* const bl = (sq & 1u) ? Al1 : Al0;
                 if constexpr (!IQN) {
@@ -2958,7 +3021,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                             }
                     }
                 }
-                if (NFB == 1u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0]);
+                if (NFB == 1u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0], ex);
                 if constexpr (Q4K) {
                     if (sq == 3) {
                         half8 fm[NB];
@@ -3040,10 +3103,16 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 const uint64_t q = q0 + m;
                 if (GATEUP && AORD == A_F32) {
                     const int e = s_rowe[m].x;
+                    uint32_t rm = 0u;
 #pragma unroll
                     for (int h = 0; h < (int)HB; ++h) {
                         const float v = swiglu(ldexpf(acc[mb][h][j], -e), ldexpf(acc[mb][HB + h][j], -e), limit);
+                        rm = max(rm, __float_as_uint(fabsf(v)));
                         if (m < n) out[q * ldo + row0 + 16u * HB * wave + 16u * h + ln] = v;
+                    }
+                    if constexpr (Q8) {
+                        rm = row_max16(rm);
+                        if (ln == 0u) rpart[wave][m] = rm;
                     }
                 } else if (GATEUP) {
                     // g, u in true units, then act 2^a_t; act column row0 + 16 HB w + 16 h + ln
@@ -3057,10 +3126,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                     uint32_t rm = __float_as_uint(fabsf(v[0]));
 #pragma unroll
                     for (int h = 1; h < (int)HB; ++h) rm = max(rm, __float_as_uint(fabsf(v[h])));
-                    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0xb1, 0xf, 0xf, false));
-                    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x4e, 0xf, 0xf, false));
-                    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x141, 0xf, 0xf, false));
-                    rm = max(rm, (uint32_t)__builtin_amdgcn_mov_dpp((int)rm, 0x140, 0xf, 0xf, false));
+                    rm = row_max16(rm);
                     if (ln == 0u) rpart[wave][m] = rm;
                     _Float16 hh[HB], ll[HB];
 #pragma unroll
@@ -3098,13 +3164,14 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                     if (m < n) {
 #pragma unroll
                         for (int nb = 0; nb < NB; ++nb)
-                            out[q * ldo + row0 + 16u * NB * wave + 16u * nb + ln] = acc[mb][nb][j];
+                            out[q * ldo + row0 + 16u * NB * wave + 16u * nb + ln] =
+                                Q8 ? ldexpf(acc[mb][nb][j], -s_rowe[m].x) : acc[mb][nb][j];
                     }
                 }
             }
-        if constexpr (GATEUP && AORD != A_F32) {
+        if constexpr (GATEUP && (AORD != A_F32 || Q8)) {
             if ((HB == 1 && out_gs != nullptr) || rowmax != nullptr) __syncthreads();
-            if constexpr (HB == 1) {
+            if constexpr (HB == 1 && !Q8) {
                 // 32-column group g of the block's 64 act columns = waves 2 g, 2 g + 1
                 if (out_gs != nullptr) {
                     const uint32_t g = tid / TT, m = tid % TT;
@@ -3203,6 +3270,23 @@ __global__ __launch_bounds__(256) void k_read16(const uint4* __restrict__ src, u
 #pragma unroll
     for (uint32_t j = 0; j < READ_UNROLL; ++j) acc ^= v[j].x ^ v[j].y ^ v[j].z ^ v[j].w;
     if (acc == 0x9e3779b9u) sink[blockIdx.x] = acc;
+}
+
+// act [rows][F] fp32 -> hi, lo f16 with act 2^e = hi + lo (+ O(2^-22 |act|)), e
+// = x_exp of the row's maximum (rowmax), natural column order; 4 values per
+// thread. Reads and writes 8 bytes per value: 2664 rows of 768 take about 4 us.
+__global__ __launch_bounds__(256) void k_split_act(const float* __restrict__ act, const uint32_t* __restrict__ rowmax,
+                                                   uint64_t n, uint32_t F, _Float16* __restrict__ hi,
+                                                   _Float16* __restrict__ lo) {
+    const uint64_t i = 4ull * ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    const float4 v = ldexp4(*reinterpret_cast<const float4*>(act + i), x_exp(__uint_as_float(rowmax[i / F])));
+    const float a[4] = {v.x, v.y, v.z, v.w};
+    _Float16 h[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) split_f16(a[j], h[j], l[j]);
+    *reinterpret_cast<uint2*>(hi + i) = make_uint2(pack_h2(h[0], h[1]), pack_h2(h[2], h[3]));
+    *reinterpret_cast<uint2*>(lo + i) = make_uint2(pack_h2(l[0], l[1]), pack_h2(l[2], l[3]));
 }
 
 // Dense token tiles for the shared expert: tile t = {0, 64 t, min(64, T - 64 t), 0}.
@@ -3416,6 +3500,15 @@ __device__ __forceinline__ uint64_t tiled_source(uint32_t kind, uint32_t r, uint
         }
         const uint32_t t = q - 1536u;
         return (t >> 1) * stride + 98u * sb + (t & 1u);
+    }
+    if (kind == 8) {
+        const uint32_t sl = r / TILE_Q80, q = r % TILE_Q80;
+        if (q < 1024u) {
+            const uint32_t l = q >> 4, b = q & 15u;
+            return (l & 15u) * stride + 68u * sl + 34u * (b >> 3) + 2u + 8u * (l >> 4) + (b & 7u);
+        }
+        const uint32_t t = q - 1024u, b = t & 3u;
+        return (t >> 2) * stride + 68u * sl + (b < 2u ? b : 32u + b);
     }
     // IQ4_NL
     const uint32_t sl = r / TILE_IQ4NL, q = r % TILE_IQ4NL;

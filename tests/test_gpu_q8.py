@@ -1,0 +1,58 @@
+"""Q8_0 on the f16 GEMM (exact int8 operands, act split by each row's own
+maximum): routed experts on small and 64-pair tiles, resident and cached, merged
+shared expert; a gated Q8_0 shared expert beside routed experts of other formats,
+whose x is stored in that format's column order; and activations of any scale,
+which raise no range flag."""
+import numpy as np
+import pytest
+
+from ingot_amd import configs as CF
+from ingot_amd.moe import IQ2_XS, IQ4_NL, Q4_K, Q6_K, Q8_0, MoeLayer
+from test_gpu_small_tiles import LOADS, routed_inputs
+from util import check_layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("F,shared", [(64, 0), (192, 192), (768, 256)])
+def test_q8_routed(gpu, oracle, F, shared):
+    H, E = 1024, len(LOADS)
+    spec = CF.make_layer(62, 0, H, E, 1, F, Q8_0, Q8_0, shared_ffn=shared)
+    blocks = spec.gate.data.reshape(-1, 34)
+    blocks[::7, :2] = 0  # zero scales
+    blocks[1::9, 2:] = 0x80  # every value -128
+    for times in (1, 2):  # 16-pair tiles; 64-pair tiles
+        x = routed_inputs(spec, [times * v for v in LOADS], H, 62 + times)
+        res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
+        out, _, _ = check_layer(res, spec, x, oracle, f"Q8_0 F={F} shared={shared} {times}x loads")
+        assert np.array_equal(out, cached(x)[0])
+        res.destroy()
+        cached.destroy()
+
+
+@pytest.mark.parametrize("gk,dk", [(IQ2_XS, IQ2_XS), (Q6_K, Q6_K), (Q4_K, Q4_K), (Q4_K, Q8_0), (IQ4_NL, IQ4_NL)])
+def test_q8_shared_beside_other_formats(gpu, oracle, gk, dk):
+    spec = CF.make_layer(63, gk, 2048, 32, 8, 512, gk, dk, shared_ffn=256, shared_gate_kind=Q8_0,
+                         shared_down_kind=Q8_0, shared_gated=True)
+    res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
+    for T in (9, 17, 130):
+        x = CF.inputs(63, T, 2048, seed=T)
+        out, _, _ = check_layer(res, spec, x, oracle, f"Q8_0 shared beside {gk}/{dk} T={T}")
+        assert np.array_equal(out, cached(x)[0])
+    res.destroy()
+    cached.destroy()
+
+
+@pytest.mark.parametrize("scale", [1e-12, 1e-4, 1e4, 1e12])
+def test_q8_any_activation_scale(gpu, oracle, scale):
+    """No token-wise guess of the activations' size enters: the relative error
+    stays that of the usual scale (two 32-bit sums of at most 1024 products)."""
+    spec = CF.make_layer(64, 0, 1024, 16, 4, 256, Q8_0, Q8_0)
+    x = (CF.inputs(64, 40, 1024) * np.float32(scale)).astype(np.float32)
+    layer = MoeLayer(gpu, spec)
+    out, ids, _ = layer(x)
+    assert not layer.last_fallback
+    st, ref, rids, _ = oracle.moe_forward(spec, x, oracle.F64)
+    assert st == 0 and np.array_equal(ids, rids)
+    assert np.linalg.norm(out - ref) <= 1e-5 * np.linalg.norm(ref)
+    layer.destroy()
