@@ -23,6 +23,9 @@ using namespace ingot;
 // (ingot_route, ingot_route_batch), word i >= 1 to the layer attached to slot
 // i, so that a check can name the layer whose kernels raised a flag.
 constexpr uint32_t FLAG_WORDS = 1024;
+// The most device memory a context keeps between ingot_moe calls: two tokens' worth of a
+// Qwen3-30B-A3B-shaped layer's selected experts; a larger call allocates and frees its own.
+constexpr uint64_t DROPIN_KEEP = 64ull << 20;
 
 struct ingot_ctx {
     int device = 0;
@@ -34,6 +37,10 @@ struct ingot_ctx {
     uint32_t* d_flags = nullptr;  // FLAG_WORDS words
     void* scratch = nullptr;  // this device's copy of `scratch` (hipGetSymbolAddress)
     hipStream_t copy = nullptr;  // cached layers' expert copies (created with the first one)
+    // Device memory kept for ingot_moe's matrices and vectors from call to call
+    // (calls on a context are one at a time and synchronous), at most DROPIN_KEEP.
+    void* dropin = nullptr;
+    uint64_t dropin_bytes = 0;
     std::vector<ingot_layer*> slot{nullptr};  // slot[i]: the live layer owning flag word i (slot 0 unused)
     uint32_t live = 0;                         // live layers on this context
     uint32_t next_seq = 0;                     // creation number of the next layer
@@ -850,6 +857,7 @@ int ingot_ctx_destroy(ingot_ctx* ctx) {
         (void)hipStreamSynchronize(ctx->copy);
         (void)hipStreamDestroy(ctx->copy);
     }
+    if (ctx->dropin) (void)hipFree(ctx->dropin);
     if (ctx->d_flags) (void)hipFree(ctx->d_flags);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
     delete ctx;
@@ -1084,38 +1092,68 @@ int ingot_moe(ingot_ctx* ctx, const ingot_matrix routed[3], const ingot_matrix* 
             (has_shared && !supported(shared_gate->kind)))
             return fail(ctx, INGOT_UNSUPPORTED, "GGML type has no kernel here");
     const uint32_t F = (uint32_t)routed[0].rows, SF = has_shared ? (uint32_t)shared[0].rows : 0;
+    // After a failed copy: no launched product may still read the memory.
+    auto drain = [ctx](int status) {
+        (void)hipStreamSynchronize(ctx->stream);
+        return status;
+    };
+    // One block of device memory: the matrices, then x[H] w[K] g,u,a [K F] y [K H]
+    // sg,su,sa [SF] sy [H] slogit [1] out [H]. (An allocation and a free per matrix
+    // took about as long as half of the copies.)
+    const ingot_matrix* src[7] = {&routed[0], &routed[1], &routed[2]};
+    uint32_t nm = 3;
+    if (has_shared) {
+        for (int i = 0; i < 3; ++i) src[nm++] = &shared[i];
+        src[nm++] = shared_gate;
+    }
+    uint64_t at[8] = {0};
+    for (uint32_t i = 0; i < nm; ++i) at[i + 1] = at[i] + ((src[i]->nbytes + 255) & ~255ull);
+    const uint64_t n = H + K + 3ull * K * F + (uint64_t)K * H + 3ull * SF + H + 1 + H, total = at[nm] + 4 * n;
     DevScope sc;
-    DevMatrix dr[3], ds[3], dg;
-    int st = INGOT_OK;
-    for (int i = 0; i < 3 && st == INGOT_OK; ++i) st = upload_scoped(ctx, sc, &routed[i], &dr[i]);
-    for (int i = 0; i < 3 && st == INGOT_OK && has_shared; ++i) st = upload_scoped(ctx, sc, &shared[i], &ds[i]);
-    if (st == INGOT_OK && has_shared) st = upload_scoped(ctx, sc, shared_gate, &dg);
-    if (st != INGOT_OK) return st;
-    // scratch: x[H] w[K] g,u,a [K F] y [K H] sg,su,sa [SF] sy [H] slogit [1] out [H]
-    const uint64_t n = H + K + 3ull * K * F + (uint64_t)K * H + 3ull * SF + H + 1 + H;
-    float* d = nullptr;
-    HIP_TRY(ctx, sc.alloc(&d, 4 * n));
+    uint8_t* base = nullptr;
+    if (total <= DROPIN_KEEP) {
+        if (total > ctx->dropin_bytes) {
+            if (ctx->dropin) HIP_TRY(ctx, hipFree(ctx->dropin));
+            ctx->dropin = nullptr;
+            ctx->dropin_bytes = 0;
+            HIP_TRY(ctx, hipMalloc(&ctx->dropin, total));
+            ctx->dropin_bytes = total;
+        }
+        base = static_cast<uint8_t*>(ctx->dropin);
+    } else {
+        HIP_TRY(ctx, sc.alloc(&base, total));
+    }
+    float* d = reinterpret_cast<float*>(base + at[nm]);
     float *dx = d, *dw = dx + H, *g = dw + K, *u = g + (uint64_t)K * F, *a = u + (uint64_t)K * F,
           *y = a + (uint64_t)K * F, *sg = y + (uint64_t)K * H, *su = sg + SF, *sa = su + SF, *sy = sa + SF,
           *sl = sy + H, *dout = sl + 1;
     hipStream_t s = ctx->stream;
-    HIP_TRY(ctx, hipMemcpy(dx, x, 4 * H, hipMemcpyHostToDevice));
-    HIP_TRY(ctx, hipMemcpy(dw, weights, 4ull * K, hipMemcpyHostToDevice));
-    auto project = [&](const DevMatrix& m, const float* in, uint64_t instride, float* o) {
+    std::vector<float> xw(x, x + H);
+    xw.insert(xw.end(), weights, weights + K);
+    HIP_TRY(ctx, hipMemcpy(dx, xw.data(), 4 * (H + K), hipMemcpyHostToDevice));
+    // Matrix i's copy (synchronous), then its product: a product runs while the next
+    // matrix is copied.
+    auto project = [&](uint32_t i, const float* in, uint64_t instride, float* o) -> int {
+        const ingot_matrix& m = *src[i];
+        HIP_TRY(ctx, hipMemcpy(base + at[i], m.data, m.nbytes, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(k_project_generic, dim3((uint32_t)((m.rows + 3) / 4), (uint32_t)m.count), dim3(256), 0, s,
-                           m.d, m.stride, m.kind, (uint32_t)m.cols, (uint32_t)m.rows, in, instride, o);
+                           base + at[i], m.stride, m.kind, (uint32_t)m.cols, (uint32_t)m.rows, in, instride, o);
+        return INGOT_OK;
     };
-    project(dr[0], dx, 0, g);
-    project(dr[1], dx, 0, u);
+    int st = project(0, dx, 0, g);
+    if (st == INGOT_OK) st = project(1, dx, 0, u);
+    if (st != INGOT_OK) return drain(st);
     hipLaunchKernelGGL(k_swiglu, dim3((uint32_t)((K * F + 255) / 256)), dim3(256), 0, s, g, u, (uint64_t)K * F, a);
-    project(dr[2], a, F, y);
     if (has_shared) {
-        project(ds[0], dx, 0, sg);
-        project(ds[1], dx, 0, su);
+        st = project(3, dx, 0, sg);
+        if (st == INGOT_OK) st = project(4, dx, 0, su);
+        if (st != INGOT_OK) return drain(st);
         hipLaunchKernelGGL(k_swiglu, dim3((SF + 255) / 256), dim3(256), 0, s, sg, su, (uint64_t)SF, sa);
-        project(ds[2], sa, SF, sy);
-        project(dg, dx, 0, sl);
+        st = project(5, sa, SF, sy);
+        if (st == INGOT_OK) st = project(6, dx, 0, sl);
     }
+    if (st == INGOT_OK) st = project(2, a, F, y);
+    if (st != INGOT_OK) return drain(st);
     hipLaunchKernelGGL(k_combine_host, dim3((uint32_t)((H + 255) / 256)), dim3(256), 0, s, y,
                        has_shared ? sy : nullptr, dw, sl, (uint32_t)H, K, dout);
     LAUNCH_CHECK(ctx);
