@@ -28,12 +28,7 @@
 
 namespace ingot {
 
-// tiles == NULL: a dense product (a shared expert beside routed experts of
-// another format), tile t = rows 16 t .. of the a_rows input rows, expert 0.
-// XORD: the column order in which x is stored where it is not the order the
-// format reads (Q8_0's natural one): the operand's pieces are then looked up in
-// it, which every order that keeps runs of 8 columns inside a superblock allows.
-template <int KIND, bool GATEUP, int AORD, bool TL, int XORD = A_NATURAL>
+template <int KIND, bool GATEUP, int AORD, bool TL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : KIND == 8 || KIND == 14 ? 3 : 4))) void k_gemm_small(
     const uint8_t* __restrict__ w0, const uint8_t* __restrict__ w1, const uint8_t* __restrict__ ws0,
     const uint8_t* __restrict__ ws1, uint32_t e_shared, uint64_t stride0, uint64_t stride1, uint32_t rows_per_expert,
@@ -47,7 +42,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
     constexpr uint32_t NW = 4;
     using BS = BStream<KIND, NB, GATEUP, TL>;
     constexpr bool Q4K = BS::Q4K, IQG = BS::IQG, IQN = BS::IQN, Q6K = BS::Q6K, Q8 = BS::Q8;
-    static_assert(XORD == A_NATURAL || (Q8 && GATEUP && XORD != A_IQ4NL), "a natural operand in another order");
     static_assert(!Q8 || !GATEUP || AORD == A_F32, "Q8_0 gate/up writes fp32 act (k_split_act)");
     __shared__ __align__(16) _Float16 As[2][8192];
     // Q4_K group sums / 32 of the chunk, f16: per superblock 16 rows x 8 groups
@@ -57,13 +51,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
     __shared__ float gpart[GATEUP ? NW : 1][TMS];
     __shared__ uint32_t rpart[GATEUP ? NW : 1][TMS];
     // tile rounds of 8, one tile per XCD, alternating direction (as k_gemm_f16)
-    const uint32_t nt = tiles ? tiles[3] : (a_rows + TMS - 1u) / TMS, slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
+    const uint32_t nt = tiles[3], slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
     const uint32_t t = ti * 8u + ((ti & 1u) ? 7u - xcd : xcd);
     if (t >= nt) return;
     const uint32_t* tile = tiles + 4u * t;
-    const uint32_t n = tiles ? tile[2] : min(TMS, a_rows - TMS * t);
+    const uint32_t n = tile[2];
     if (n == 0) return;
-    const uint32_t e = tiles ? tile[0] : 0u, q0 = tiles ? tile[1] : TMS * t;
+    const uint32_t e = tile[0], q0 = tile[1];
     const uint32_t ew = slot_of ? slot_of[e] : e;  // cached experts, as in k_gemm_f16
     if (ew == NO_SLOT) return;
     const uint32_t row0 = (slot - ti * nblk) * (GATEUP ? 64u : 128u);
@@ -202,8 +196,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
                 }
 #pragma unroll
                 for (uint32_t gi = 0; gi < 2; ++gi) {
-                    const uint32_t cn = 32u * PART + 8u * sq + (IQG ? 2u * kq + gi : 4u * gi + kq);
-                    const uint32_t ch = XORD == A_NATURAL ? cn : a_pos<XORD>(8u * cn) >> 3;
+                    const uint32_t ch = 32u * PART + 8u * sq + (IQG ? 2u * kq + gi : 4u * gi + kq);
                     const half8 a0 = *reinterpret_cast<const half8*>(&A[ln * CH + 8u * (ch ^ ln)]);
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb) {

@@ -188,8 +188,8 @@ bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, 
 
 template <int KIND, bool GATEUP>
 void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a) {
-#define SML_(AO, TLV, ...)                                                                                       \
-    hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV, ##__VA_ARGS__>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
+#define SML_(AO, TLV)                                                                                            \
+    hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
                        a.e_shared, a.stride0, a.stride1, a.rows_per_expert, a.kdim, a.ah, a.al, a.gs, a.pairs,   \
                        a.K, a.tiles, a.ldo, a.limit, a.out, a.out_h, a.out_l, a.out_gs, a.nblk, a.a_rows,        \
                        a.xstat, a.rowmax, a.flags, a.slot_of)
@@ -200,11 +200,7 @@ void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const Gemm
         return;                 \
     } while (0)
     if constexpr (GATEUP && KIND == 8) {
-        // act in fp32; aord is the order in which x is stored (a dense product reads
-        // GGUF order, the routed experts' x is natural)
-        if (aord == A_IQ3XXS) SML_(A_F32, false, A_IQ3XXS);
-        else if (aord == A_Q6K) SML_(A_F32, false, A_Q6K);
-        else SML(A_F32);
+        SML(A_F32);
     } else if constexpr (GATEUP) {
         switch (aord) {
             case A_IQ4NL: SML(A_IQ4NL);

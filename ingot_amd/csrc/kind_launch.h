@@ -137,10 +137,15 @@ struct GemmF16Args {
 // always), else 64; false if no instantiation covers the arguments.
 template <int KIND, bool GATEUP>
 bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, const GemmF16Args& a);
-// k_gemm_small<KIND, GATEUP, aord, tl>: the same over tiles of at most TMS pairs
-// (Q8_0 gate/up: aord is the column order of x).
+// k_gemm_small<KIND, GATEUP, aord, tl>: the same over tiles of at most TMS pairs.
 template <int KIND, bool GATEUP>
 void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const GemmF16Args& a);
+
+// k_dense_q8: a Q8_0 shared expert's gate/up (x in column order xord; act in fp32,
+// row maxima in rowmax) and down products over T tokens.
+void launch_dense_q8(hipStream_t s, bool gateup, int xord, const uint8_t* w0, const uint8_t* w1, uint64_t stride0,
+                     uint64_t stride1, uint32_t rows, uint32_t kdim, const _Float16* ah, const _Float16* al, uint32_t T,
+                     float limit, float* out, const float* xstat, uint32_t* rowmax);
 
 #define INGOT_DECLARE_F16(K)                                                                                \
     extern template bool launch_gemm_f16_k<K, true>(hipStream_t, int, bool, bool, dim3, const GemmF16Args&); \

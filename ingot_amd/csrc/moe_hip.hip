@@ -740,12 +740,12 @@ static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
     p.merge = p.f16 && L->has_shared && L->SF == L->F && L->sgate.kind == L->gate.kind &&
               L->sup.kind == L->up.kind && L->sdown.kind == L->down.kind && L->sgate.stride == L->gate.stride &&
               L->sup.stride == L->up.stride && L->sdown.stride == L->down.stride;
-    // A Q8_0 shared expert that does not join: k_gemm_small over dense tiles, where
-    // x is stored in an order it can look up; rows P .. of acth / actl hold its act.
-    // (512 experts, IQ2_XS, at 509 tokens: 64 + 128 blocks of the fp32 GEMM took 55
-    // and 14 us.)
+    // A Q8_0 shared expert that does not join: k_dense_q8, where x is stored in an
+    // order it can look up; rows P .. of acth / actl hold its act. 512 x 2048, gate/up +
+    // down us, fp32 GEMM (whose 64-token tiles give few blocks) against it: 60 / 17 at 8
+    // tokens, 69 / 57 at 509, about 85 / 200 at 2048.
     p.dense8 = p.f16gu && L->has_shared && !p.merge && L->sgate.kind == 8 && L->sdown.kind == 8 && L->SF <= L->F &&
-               a_order(L->gate.kind) != A_IQ4NL;
+               T <= 640 && a_order(L->gate.kind) != A_IQ4NL;
     return p;
 }
 
@@ -1605,7 +1605,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         const PrefillPlan plan = prefill_plan(L, T);
         const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge, dense8 = plan.dense8;
         const bool q8 = f16 && gate.kind == 8;
-        const int xord = a_order(gate.kind), aord = q8 ? xord : f16 ? a_order(down.kind) : A_F32;
+        const int xord = a_order(gate.kind), aord = f16 ? a_order(down.kind) : A_F32;
         const bool mins = f16 && (down.kind == 12 || down.kind == 13);
         // 128-token tiles when an expert can take more than 64 pairs (each takes at
         // most one per token), the launch averages at least 32 pairs per expert
@@ -1646,7 +1646,6 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             const uint64_t n = rows * f;
             hipLaunchKernelGGL(k_split_act, dim3((uint32_t)((n / 4 + 255) / 256)), dim3(256), 0, ss, a, rm, n, f, h, l);
         };
-        auto dense_grid = [T](uint32_t nblk) { return dim3(8 * nblk * (((T + TMS - 1) / TMS + 7) / 8)); };
         // Dispatch stage: expert grouping, and for the f16 GEMM the split of x
         // into f16 hi/lo with its 32-column sums.
         L->stage[ST_DISPATCH] = [=](hipStream_t ss) {
@@ -1683,13 +1682,8 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             }
             if (q8) split_act(ss, act, rmx, (uint64_t)(P + S), F, acth, actl);
             if (dense8 && LL->pass.first) {
-                launch_gemm_small<true>(ss, 8u, xord, false, dense_grid(SF / 64), (const uint8_t*)sgate.d,
-                                        (const uint8_t*)sup.d, (const uint8_t*)nullptr, (const uint8_t*)nullptr,
-                                        0xffffffffu, sgate.stride, sup.stride, SF, H, (const _Float16*)xh,
-                                        (const _Float16*)xl, (const float*)nullptr, (const uint32_t*)nullptr, 1u,
-                                        (const uint32_t*)nullptr, SF, limit, sact, (_Float16*)nullptr,
-                                        (_Float16*)nullptr, (float*)nullptr, SF / 64, T, (const float*)xstat,
-                                        rowmax + P, flags, (const uint32_t*)nullptr);
+                launch_dense_q8(ss, true, xord, sgate.d, sup.d, sgate.stride, sup.stride, SF, H, xh, xl, T, limit, sact,
+                                xstat, rowmax + P);
             } else if (hs && !merge && LL->pass.first)
                 launch_gemm<true>(ss, sgate.kind, dim3(SF / 64, scap), sgate.d, sup.d, sgate.stride, sup.stride, SF, H,
                                   xin, nullptr, 1, stiles, SF, limit, sact);
@@ -1717,13 +1711,8 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             if (dense8 && LL->pass.first) {
                 _Float16 *sh = acth + (uint64_t)P * F, *sl = actl + (uint64_t)P * F;
                 split_act(ss, sact, rowmax + P, T, SF, sh, sl);
-                launch_gemm_small<false>(ss, 8u, A_NATURAL, false, dense_grid(H / 128), (const uint8_t*)sdown.d,
-                                         (const uint8_t*)nullptr, (const uint8_t*)nullptr, (const uint8_t*)nullptr,
-                                         0xffffffffu, sdown.stride, 0ull, H, SF, (const _Float16*)sh,
-                                         (const _Float16*)sl, (const float*)nullptr, (const uint32_t*)nullptr, 1u,
-                                         (const uint32_t*)nullptr, H, 0.f, Ys, (_Float16*)nullptr, (_Float16*)nullptr,
-                                         (float*)nullptr, H / 128, T, (const float*)xstat, rowmax + P, flags,
-                                         (const uint32_t*)nullptr);
+                launch_dense_q8(ss, false, A_NATURAL, sdown.d, nullptr, sdown.stride, 0ull, H, SF, sh, sl, T, 0.f, Ys,
+                                xstat, rowmax + P);
             } else if (hs && !merge && LL->pass.first)
                 launch_gemm<false>(ss, sdown.kind, dim3(H / 128, scap), sdown.d, nullptr, sdown.stride, 0, H, SF, sact,
                                    nullptr, 1, stiles, H, 0.f, Ys);

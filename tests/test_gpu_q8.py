@@ -35,7 +35,7 @@ def test_q8_shared_beside_other_formats(gpu, oracle, gk, dk):
     spec = CF.make_layer(63, gk, 2048, 32, 8, 512, gk, dk, shared_ffn=256, shared_gate_kind=Q8_0,
                          shared_down_kind=Q8_0, shared_gated=True)
     res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
-    for T in (9, 17, 130):
+    for T in (9, 17, 130, 300):  # one and four 16-token tiles per block
         x = CF.inputs(63, T, 2048, seed=T)
         out, _, _ = check_layer(res, spec, x, oracle, f"Q8_0 shared beside {gk}/{dk} T={T}")
         assert np.array_equal(out, cached(x)[0])
