@@ -192,7 +192,7 @@ void launch_gemm_small_k(hipStream_t s, int aord, bool tl, dim3 grid, const Gemm
     hipLaunchKernelGGL((k_gemm_small<KIND, GATEUP, AO, TLV>), grid, dim3(256), 0, s, a.w0, a.w1, a.ws0, a.ws1,   \
                        a.e_shared, a.stride0, a.stride1, a.rows_per_expert, a.kdim, a.ah, a.al, a.gs, a.pairs,   \
                        a.K, a.tiles, a.ldo, a.limit, a.out, a.out_h, a.out_l, a.out_gs, a.nblk, a.a_rows,        \
-                       a.xstat, a.rowmax, a.flags, a.slot_of)
+                       a.xstat, a.rowmax, a.flags, a.slot_of, a.flat)
 #define SML(AO)                 \
     do {                        \
         if (tl) SML_(AO, true); \

@@ -1626,6 +1626,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         // in w.acts, the group sums that only Q4_K and Q5_K use).
         const uint32_t pcap = (P + TMS - 1) / TMS + E + (merge ? (T + TMS - 1) / TMS : 0u);
         const bool small = f16 && P <= SMALL_PAIRS_PER_EXPERT * E && 16ull * pcap <= (q8 ? 4ull * P * (F / 32) : 4ull * P * F);
+        const uint32_t flat = P <= 8u * E ? 1u : 0u;
         uint32_t* const ptiles = small ? reinterpret_cast<uint32_t*>(q8 ? w.acts : w.act) : nullptr;
         const uint32_t tm = tt128 ? 2u * TM : TM;
         const uint8_t *g16 = tlg ? gate.t : gate.d, *u16 = tlg ? up.t : up.d, *d16 = tld ? down.t : down.d;
@@ -1668,7 +1669,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                         H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
                                         (const uint32_t*)pairs, K, (const uint32_t*)ptiles, F, limit, q8 ? act : (float*)nullptr,
                                         acth, actl, mins ? acts : nullptr, F / 64, T, (const float*)xstat, rmx, flags,
-                                        so);
+                                        so, flat);
             } else if (f16gu) {
                 launch_gemm_f16<true>(ss, gate.kind, aord, tt128, tlg, dim3(8 * (F / 64) * ((capf + 7) / 8)), g16, u16,
                                       merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride,
@@ -1697,7 +1698,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                          down.stride, 0ull, H, F, (const _Float16*)acth, (const _Float16*)actl,
                                          (const float*)acts, (const uint32_t*)nullptr, K, (const uint32_t*)ptiles, H, 0.f,
                                          Y, (_Float16*)nullptr, (_Float16*)nullptr, (float*)nullptr, H / 128,
-                                         (uint32_t)(P + S), (const float*)xstat, rmx, flags, so);
+                                         (uint32_t)(P + S), (const float*)xstat, rmx, flags, so, flat);
             else if (f16)
                 launch_gemm_f16<false>(ss, down.kind, A_NATURAL, tt128, tld, dim3(8 * (H / 128) * ((capf + 7) / 8)), d16,
                                        (const uint8_t*)nullptr, merge ? sd16 : nullptr, (const uint8_t*)nullptr, e_sh,
