@@ -657,6 +657,9 @@ static uint64_t carve(const ingot_layer* L, uint32_t T, void* base, Ws* out) {
     Ws w;
     w.stile_cap = (T + TM - 1) / TM;
     w.tile_cap = (uint32_t)((P + TM - 1) / TM + L->E + (L->SF ? w.stile_cap : 0));
+    // act and sact are one part: a merged Q8_0 shared expert's gate/up writes its fp32
+    // act as rows P..P+T-1 of act (F == SF), which are sact's.
+    const uint64_t act_bytes = 4ull * P * L->F;  // F % 64 == 0: keeps sact 256-byte aligned
     struct Part {
         void** p;
         uint64_t bytes;
@@ -664,8 +667,7 @@ static uint64_t carve(const ingot_layer* L, uint32_t T, void* base, Ws* out) {
     const Part parts[] = {
         {(void**)&w.xn, 4ull * T * L->H},       {(void**)&w.logits, 4ull * T * L->E},
         {(void**)&w.sgl, 4ull * T},             {(void**)&w.ids, 4ull * P},
-        {(void**)&w.wts, 4ull * P},             {(void**)&w.act, 4ull * P * L->F},
-        {(void**)&w.sact, 4ull * T * (L->SF ? L->SF : 1)},
+        {(void**)&w.wts, 4ull * P},             {(void**)&w.act, act_bytes + 4ull * T * (L->SF ? L->SF : 1)},
         {(void**)&w.Y, 4ull * PS * L->H},
         {(void**)&w.counts, 4ull * L->E},       {(void**)&w.first, 4ull * L->E},
         {(void**)&w.tiles, 16ull * w.tile_cap}, {(void**)&w.pairs, 4ull * PS},
@@ -682,6 +684,7 @@ static uint64_t carve(const ingot_layer* L, uint32_t T, void* base, Ws* out) {
         *p.p = base ? static_cast<char*>(base) + off : nullptr;
         off += (p.bytes + 255) & ~255ull;
     }
+    w.sact = base ? w.act + act_bytes / 4 : nullptr;
     if (out) *out = w;
     return off;
 }
