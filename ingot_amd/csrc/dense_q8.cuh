@@ -65,7 +65,7 @@ __global__ __launch_bounds__(256) void k_dense_q8(const uint8_t* __restrict__ w0
     for (uint32_t sb = wave; sb < nsb; sb += NW) {
         Frag f[AHEAD];
 #pragma unroll
-        for (uint32_t s = 0; s < 4u; ++s) B.load_slab(s, 4u * sb + s);
+        for (uint32_t s = 0; s < 4u; ++s) B.load_slab(s, 4u * sb + s, (s & 1u) == 0u);
 #pragma unroll
         for (uint32_t s = 0; s < AHEAD; ++s) load_a(f[s], sb, s);
 #pragma unroll
@@ -73,7 +73,8 @@ __global__ __launch_bounds__(256) void k_dense_q8(const uint8_t* __restrict__ w0
             half8 fb[NB][2], fe[NB][2];
             float dg[NB][2];
             typename BStream<8, NB, GATEUP, false>::SbState st;
-            B.decode(st, s, B.nq[s], B.nd[s], fb, dg, fe, B.n1[s]);
+            if ((s & 1u) == 0u) B.take_pair(s);
+            B.decode(st, s, B.nq[s], B.nd[s], fb, dg, fe);
             // (slabs past K: clamped weights over columns past it, not added)
             const bool live = 4u * sb + s < slabs;
 #pragma unroll

@@ -184,18 +184,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!TL ? 2 : K
                 const uint32_t s = 4u * sb + sq;
                 // B of slab s out of the ring, B(s + DEPTH) into its slot
                 uint4 qv[NB];
-                uint32_t ex[NB];
                 uint2 dv[NB];
+                if ((sq & 1u) == 0u) B.take_pair(sq);
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     qv[nb] = B.nq[sq][nb];
                     if constexpr (IQN && !Q8) qv[nb].z = B.n1[sq][nb];
-                    if constexpr (Q8) ex[nb] = B.n1[sq][nb];
                     if constexpr (IQN || Q6K) dv[nb] = B.nd[sq][nb];
                 }
                 half8 fb[NB][2], fe[NB][2];
                 float dg[NB][2];
-                B.decode(cur, sq, qv, dv, fb, dg, fe, ex);
+                B.decode(cur, sq, qv, dv, fb, dg, fe);
                 B.load_slab(sq, s + DEPTH, (sq & 1u) == 0u);
                 if constexpr (!IQN) {
                     if (sq == 0) B.load_hdr(sb + 1u);

@@ -2278,8 +2278,19 @@ struct BStream {
     uint4 nq[4][NB];
     uint32_t n1[4][NB];
     uint2 nd[4][NB];
+    // Q8_0 in GGUF order (34-byte blocks) is loaded two slabs at a time: lane 16 kq + ln
+    // takes the whole of block kq of row ln's four, so that each byte is read once, and
+    // take_pair hands each lane its 8 columns of every block. (Loads of what each lane
+    // decodes, four a slab, touch every line of 16 rows about eight times, and the rows
+    // of a CU's waves are more lines than its L1 holds.) Gate/up + down of 128 experts
+    // of 768 x 2048 at 32 / 160 / 333 / 4096 tokens: four loads a slab 279 / 340 / 444 /
+    // 1524 us, pairs 155 / 193 / 256 / 1078; the fp32 GEMM 249 / 288 / 387 / 2680, the
+    // tiled copy 117 / 145 / 183 / 906.
+    static constexpr bool Q8P = Q8 && !TL;
+    uint32_t raw[Q8P ? 2 : 1][Q8P ? NB : 1][9];
     // Q6_K: ev (the slab is the first of its half, a compile-time constant at
-    // each call) also loads the half's qh window.
+    // each call) also loads the half's qh window. Q8_0 in GGUF order: ev loads the
+    // pair of slabs into raw[rs / 2].
     __device__ __forceinline__ void load_slab(uint32_t rs, uint32_t s, bool ev = false) {
         s = s < slabs ? s : slabs - 1u;
 #pragma unroll
@@ -2341,13 +2352,17 @@ struct BStream {
                 nq[rs][nb] = buf_load16(rw, 16u * lane, u);
                 nd[rs][nb].x = buf_load4(rw, 4u * ln, u + 1024u);
             } else if constexpr (Q8) {
-                // the first block's bytes 2 bytes off a dword, the second's on one
-                const uint32_t u = bsoff[nb] + 68u * s;
-                const auto a = __builtin_amdgcn_raw_buffer_load_b96(rw, (int)(boff[nb] + 8u * kq), (int)u, 0);
-                const uint2 b = buf_load8(rw, boff[nb] + 8u * kq, u + 36u);
-                nq[rs][nb] = make_uint4(a[0], a[1], b.x, b.y);
-                n1[rs][nb] = a[2];
-                nd[rs][nb] = make_uint2(buf_load4(rw, boff[nb], u), buf_load4(rw, boff[nb], u + 32u));
+                // 36 bytes from the dword at or before the block: one in an even place
+                // starts on a dword, one in an odd place 2 bytes later. (Past K: the row's
+                // last block, always in an odd place, whose 36 bytes end with it.)
+                if (ev) {
+                    const uint32_t b = min(2u * s + kq, 2u * slabs - 1u), v = boff[nb] + 34u * b - 2u * (b & 1u);
+                    uint32_t* const r = raw[rs >> 1][nb];
+                    const uint4 a = buf_load16(rw, v, bsoff[nb]), c = buf_load16(rw, v, bsoff[nb] + 16u);
+                    r[0] = a.x, r[1] = a.y, r[2] = a.z, r[3] = a.w;
+                    r[4] = c.x, r[5] = c.y, r[6] = c.z, r[7] = c.w;
+                    r[8] = buf_load4(rw, v, bsoff[nb] + 32u);
+                }
             } else if constexpr (IQ4) {
                 const uint32_t u = bsoff[nb] + 36u * s;
                 const uint2 q = buf_load8(rw, boff[nb] + 4u * kq, u);
@@ -2355,6 +2370,38 @@ struct BStream {
                 nq[rs][nb].y = q.y;
                 n1[rs][nb] = buf_load4(rw, boff[nb] + 4u * kq, u + 20u);
                 nd[rs][nb] = make_uint2(buf_load4(rw, boff[nb], u), buf_load4(rw, boff[nb], u + 16u));
+            }
+        }
+    }
+    // Q8_0 in GGUF order: the pair of slabs in raw[rs / 2] into ring slots rs, rs + 1 (rs
+    // even), as load_slab leaves a tiled slab. Lane group kq holds 8-column chunks 0..3
+    // of block kq and takes chunk kq of blocks 0..3: a 4 x 4 transpose over the groups.
+    __device__ __forceinline__ void take_pair(uint32_t rs) {
+        if constexpr (Q8P) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) {
+                const uint32_t* const r = raw[rs >> 1][nb];
+                const uint32_t sel = (kq & 1u) ? 0x07060504u : 0x05040302u;
+                uint32_t c[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) c[i] = __builtin_amdgcn_perm(r[i + 1], r[i], sel);
+                const uint32_t d = (kq & 1u) ? r[0] >> 16 : r[0] & 0xffffu;
+                uint32_t o[4][2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const auto a = __builtin_amdgcn_permlane32_swap(c[j], c[4 + j], false, false);
+                    const auto b = __builtin_amdgcn_permlane32_swap(c[2 + j], c[6 + j], false, false);
+                    const auto lo = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+                    const auto hi = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+                    o[0][j] = lo[0], o[1][j] = lo[1], o[2][j] = hi[0], o[3][j] = hi[1];
+                }
+                const auto dd = __builtin_amdgcn_permlane32_swap(d, d, false, false);
+                const auto dl = __builtin_amdgcn_permlane16_swap(dd[0], dd[0], false, false);
+                const auto dh = __builtin_amdgcn_permlane16_swap(dd[1], dd[1], false, false);
+                nq[rs][nb] = make_uint4(o[0][0], o[0][1], o[1][0], o[1][1]);
+                nd[rs][nb].x = dl[0] | (dl[1] << 16);
+                nq[rs + 1u][nb] = make_uint4(o[2][0], o[2][1], o[3][0], o[3][1]);
+                nd[rs + 1u][nb].x = dh[0] | (dh[1] << 16);
             }
         }
     }
@@ -2477,8 +2524,7 @@ struct BStream {
     // into fb, B_e into fe); IQ4_NL also yields the units of its two blocks and
     // whether a d is zero.
     __device__ __forceinline__ void decode(const SbState& st, uint32_t sq, const uint4* qv, const uint2* dv,
-                                           half8 (*fb)[2], float (*dg)[2], half8 (*fe)[2],
-                                           const uint32_t* ex = nullptr) {
+                                           half8 (*fb)[2], float (*dg)[2], half8 (*fe)[2]) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             if constexpr (Q6K) {
@@ -2623,12 +2669,8 @@ struct BStream {
                 }
             } else if constexpr (Q8) {
                 // int8 q -> f16 bits 0x6400 | (q ^ 0x80) = 1152 + q, minus 1152
-                const float d[2] = {half_bits_to_float(dv[nb].x & 0xffffu),
-                                    half_bits_to_float((TL ? dv[nb].x : dv[nb].y) >> 16)};
-                // (GGUF order: the first block's bytes from their window, its third word in ex)
-                const uint32_t w[4] = {TL ? qv[nb].x : __builtin_amdgcn_alignbit(qv[nb].y, qv[nb].x, 16u),
-                                       TL ? qv[nb].y : __builtin_amdgcn_alignbit(ex[nb], qv[nb].y, 16u), qv[nb].z,
-                                       qv[nb].w};
+                const float d[2] = {half_bits_to_float(dv[nb].x & 0xffffu), half_bits_to_float(dv[nb].x >> 16)};
+                const uint32_t w[4] = {qv[nb].x, qv[nb].y, qv[nb].z, qv[nb].w};
 #pragma unroll
                 for (int gi = 0; gi < 2; ++gi) {
                     uint32_t b[4];
@@ -2858,7 +2900,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     };
     // Vector-memory loads issued after a slab's A DMA: the B ring's, and at a
     // superblock's first slab its header (and Q4_K group sums).
-    constexpr uint32_t B_PER_SLAB = Q4K ? NB : IQ4 || Q8 ? (TL ? 2u : 4u) * NB : IQ4X ? (TL ? 2u : 3u) * NB : 0u;
+    constexpr uint32_t B_PER_SLAB = Q4K ? NB : IQ4 ? (TL ? 2u : 4u) * NB : Q8 ? 2u * NB : IQ4X ? (TL ? 2u : 3u) * NB : 0u;
     constexpr uint32_t B_PER_SB = Q5K                ? 2u * NB + 1u
                                   : Q4K              ? NB + 1u
                                   : IQ2S             ? (TL ? 3u : 7u) * NB
@@ -2909,17 +2951,16 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
         float dgs[NFB][NB][2];
         {
             uint4 qv[NB];
-            uint32_t ex[NB];
             uint2 dv[NB];
+            B.take_pair(0);
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
                 qv[nb] = B.nq[0][nb];
                 if constexpr (IQN && !Q8) qv[nb].z = B.n1[0][nb];
-                if constexpr (Q8) ex[nb] = B.n1[0][nb];
                 if constexpr (IQN || Q6K) dv[nb] = B.nd[0][nb];
             }
             B.load_slab(0, DEPTH, true);
-            B.decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0], ex);
+            B.decode(cur, 0u, qv, dv, fb[0], dgs[0], fe[0]);
         }
         for (uint32_t s0 = 0; s0 < slabs; s0 += UNR) {
             const uint32_t sb = s0 >> 2;
@@ -2942,13 +2983,12 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 // B of slab s + 1 out of the ring, B(s + 1 + DEPTH) into its slot.
                 const uint32_t rs = (sq + 1u) % DEPTH;
                 uint4 qv[NB];
-                uint32_t ex[NB];
                 uint2 dv[NB];
+                if (sq & 1u) B.take_pair(rs);
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) {
                     qv[nb] = B.nq[rs][nb];
                     if constexpr (IQN && !Q8) qv[nb].z = B.n1[rs][nb];
-                    if constexpr (Q8) ex[nb] = B.n1[rs][nb];
                     if constexpr (IQN || Q6K) dv[nb] = B.nd[rs][nb];
                 }
                 // (s is a multiple of UNR plus sq: slab s + 1 + DEPTH opens a half when sq is odd)
@@ -2968,7 +3008,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                 const uint32_t cb = NFB == 2u ? (sq & 1u) : 0u, nb_ = NFB == 2u ? cb ^ 1u : 0u;
                 // (after the last slab: a decode of clamped bytes that nothing reads;
                 // kept unconditional so that the decode shares a block with the MFMAs)
-                if (NFB == 2u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u], ex);
+                if (NFB == 2u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[nb_], dgs[nb_], fe[Q6K ? nb_ : 0u]);
                 const _Float16* const bh = (sq & 1u) ? Ah1 : Ah0;
                 const _Float16* const bl = (sq & 1u) ? Al1 : Al0;
                 if constexpr (!IQN) {
@@ -3045,7 +3085,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                             }
                     }
                 }
-                if (NFB == 1u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0], ex);
+                if (NFB == 1u) B.decode(sq == 3 ? nxt : cur, (sq + 1u) & 3u, qv, dv, fb[0], dgs[0], fe[0]);
                 if constexpr (Q4K) {
                     if (sq == 3) {
                         half8 fm[NB];
@@ -3105,6 +3145,10 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
                     if (sq == 0) wait_vmcnt<NB + B_PER_SB>();
                     else if (sq & 1u) wait_vmcnt<2u * NB>();
                     else wait_vmcnt<NB>();
+                } else if constexpr (BS::Q8P) {
+                    // a pair of slabs at odd sq
+                    if (sq & 1u) wait_vmcnt<3u * NB>();
+                    else wait_vmcnt<0>();
                 } else if (sq == 0 && !IQN) wait_vmcnt<B_PER_SLAB + B_PER_SB>();
                 else wait_vmcnt<B_PER_SLAB>();
             }
