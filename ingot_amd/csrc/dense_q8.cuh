@@ -2,13 +2,12 @@
 // f16 MFMA (numerics as k_gemm_f16: A split hi + lo, B the int8 value, fp32 sums).
 //
 // The matrices are small (1 MB of gate and up at 512 x 2048), so what bounds a
-// batch is one wave's chain through K, about 1 us per 64 columns of GGUF-order
-// blocks read row by row. A block is therefore one 16-row block (down: two) of one
-// tile of 16 tokens with K split over its 4 waves, superblock by superblock; a
-// superblock's weights (and with one tile its A operands) are all loaded before the
-// first is used, and the waves' sums meet in LDS. 512 x 2048 gate/up at 8 / 100 / 509
-// tokens: 12 / 17 / 39 us, against 34 / 40 / 42 on k_gemm_small (K in one chain) and
-// about 55 on the fp32 GEMM.
+// batch is one wave's chain through K. A block is therefore one 16-row block (down:
+// two) of one tile of 16 tokens (or of four: launch_dense_q8) with K split over its 4
+// waves, superblock by superblock; a superblock's weights (and with one tile its A
+// operands) are all loaded before the first is used, and the waves' sums meet in LDS.
+// 512 x 2048 at 65 / 130 / 509 tokens, gate/up 12 / 16 / 27 us and down 8 / 10 / 17 (with
+// the split of act), against 86 / 86 / 88 and 25 / 26 / 26 on the fp32 GEMM.
 #pragma once
 #include "moe_kernels.cuh"
 

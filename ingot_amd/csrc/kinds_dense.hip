@@ -15,11 +15,15 @@ namespace ingot {
 void launch_dense_q8(hipStream_t s, bool gateup, int xord, const uint8_t* w0, const uint8_t* w1, uint64_t stride0,
                      uint64_t stride1, uint32_t rows, uint32_t kdim, const _Float16* ah, const _Float16* al, uint32_t T,
                      float limit, float* out, const float* xstat, uint32_t* rowmax) {
-    // One tile per block (more blocks) up to 256 tokens, four above (weights read and
-    // decoded a quarter as often): 512 x 2048 gate/up us, one against four, 17 / 30 at
-    // 100 and 130 tokens, 52 / 39 at 509.
-    const uint32_t mt = T <= 256u ? 1u : 4u;
-    const dim3 grid(rows / (gateup ? 16u : 32u), (T + 16u * mt - 1u) / (16u * mt));
+    // Four tiles per block (weights read and decoded a quarter as often, but one block
+    // per CU) where those blocks fill the rounds they take of the 256 CUs to 85 %, else one (three per
+    // CU). Gate/up stage us, one against four: 512 x 2048 at 400 / 509 / 640 tokens (224,
+    // 256, 320 blocks of four) 57 / 63 / 72 against 52 / 58 / 83; 1408 x 4096 at 256 / 509
+    // (352, 704) 123 / 203 against 129 / 191; down at H = 2048, K = 1024, 256 / 320 (256,
+    // 320) 30 / 32 against 27 / 37.
+    const uint32_t br = gateup ? 16u : 32u, b4 = rows / br * ((T + 63u) / 64u);
+    const uint32_t mt = 100u * b4 >= 85u * 256u * ((b4 + 255u) / 256u) ? 4u : 1u;
+    const dim3 grid(rows / br, (T + 16u * mt - 1u) / (16u * mt));
 #define DQ_(GU, XO, MT)                                                                                       \
     hipLaunchKernelGGL((k_dense_q8<GU, XO, MT>), grid, dim3(256), 0, s, w0, w1, stride0, stride1, rows, kdim, \
                        ah, al, T, limit, out, xstat, rowmax)

@@ -728,8 +728,12 @@ static bool f16_gemm_fits(uint64_t kdim, uint64_t rows) { return 2ull * kdim * r
 // fp32 act for the fp32 down GEMM); f16: down too; merge: the shared expert
 // joins the same launches (its formats and width equal the routed experts').
 struct PrefillPlan {
-    bool f16gu = false, f16 = false, merge = false, dense8 = false;
+    bool f16gu = false, f16 = false, merge = false;
+    bool gu8 = false, dn8 = false;  // a Q8_0 shared expert's gate/up, down on k_dense_q8
 };
+
+// Whether that many blocks, one per CU at a time, use over `percent` of the rounds they take.
+static bool fills(uint64_t blocks, uint64_t percent) { return 100 * blocks > percent * ((blocks + 255) / 256 * 256); }
 
 static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
     PrefillPlan p;
@@ -744,11 +748,26 @@ static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
               L->sup.kind == L->up.kind && L->sdown.kind == L->down.kind && L->sgate.stride == L->gate.stride &&
               L->sup.stride == L->up.stride && L->sdown.stride == L->down.stride;
     // A Q8_0 shared expert that does not join: k_dense_q8, where x is stored in an
-    // order it can look up; rows P .. of acth / actl hold its act. 512 x 2048, gate/up +
-    // down us, fp32 GEMM (whose 64-token tiles give few blocks) against it: 60 / 17 at 8
-    // tokens, 69 / 57 at 509, about 85 / 200 at 2048.
-    p.dense8 = p.f16gu && L->has_shared && !p.merge && L->sgate.kind == 8 && L->sdown.kind == 8 && L->SF <= L->F &&
-               T <= 640 && a_order(L->gate.kind) != A_IQ4NL;
+    // order it can look up; rows P .. of acth / actl hold its act. Its time grows with
+    // T x SF, the fp32 GEMM's with the rounds of its 64-token blocks over the CUs (SF / 64
+    // gate/up blocks a tile, H / 128 down), so it is taken while those leave CUs idle.
+    // Stage us with the routed experts' small part, fp32 GEMM against k_dense_q8, gate/up:
+    // 512 x 2048 at 65 / 1024 tokens (16, 128 blocks) 102 / 133 against 29 / 93; 1536 x 2048
+    // at 509 / 640 / 768 (192, 240, 288) 121 / 125 / 185 against 115 / 138 / 163; 1536 x
+    // 4096 at 320 / 640 / 2048 (120, 240, 768) 213 / 228 / 550 against 135 / 233 / 610. Down,
+    // whose K is SF (one chain of SF / 256 superblocks, and a split of act before it):
+    // 512 wide at H = 2048, 640 / 1024 / 2048 tokens (160, 256, 512 blocks) 38 / 43 / 63
+    // against 35 / 44 / 71; 64 wide at 65 / 509 (32, 128) 11 / 15 against 10 / 21; 1536 wide
+    // at H = 4096, 320 / 640 / 1024 (160, 320, 512) 86 / 135 / 145 against 64 / 100 / 151.
+    // The down product takes it after the gate/up product only (for the row maxima), so
+    // a nearly full gate/up round is given up where the down product gains more.
+    if (p.f16gu && L->has_shared && !p.merge && L->sgate.kind == 8 && L->sdown.kind == 8 && L->SF <= L->F &&
+        a_order(L->gate.kind) != A_IQ4NL) {
+        const uint64_t tt = (T + TM - 1) / TM, gu = tt * (L->SF / 64), dn = tt * (L->H / 128);
+        p.dn8 = dn <= 256 ? 2 * dn <= L->SF : L->SF >= 512 && !fills(dn, 80);
+        p.gu8 = !fills(gu, p.dn8 ? 95 : 80);
+        p.dn8 = p.dn8 && p.gu8;
+    }
     return p;
 }
 
@@ -1606,7 +1625,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         // f16 GEMM writing fp32 act and the down projection on the fp32 GEMM,
         // over the same 64-token tiles.
         const PrefillPlan plan = prefill_plan(L, T);
-        const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge, dense8 = plan.dense8;
+        const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge, gu8 = plan.gu8, dn8 = plan.dn8;
         const bool q8 = f16 && gate.kind == 8;
         const int xord = a_order(gate.kind), aord = f16 ? a_order(down.kind) : A_F32;
         const bool mins = f16 && (down.kind == 12 || down.kind == 13);
@@ -1638,8 +1657,8 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         _Float16 *xh = w.xh, *xl = w.xl, *acth = w.acth, *actl = w.actl;
         float *xs = w.xs, *acts = w.acts;
         // rows whose maxima the f16 gate/up raises (act split in the f16 GEMM's units)
-        uint32_t *rmx = f16 ? rowmax : nullptr, *rmz = f16 || dense8 ? rowmax : nullptr;
-        const uint32_t nrow = rmz ? P + (merge || dense8 ? T : 0u) : 0u;
+        uint32_t *rmx = f16 ? rowmax : nullptr, *rmz = f16 || gu8 ? rowmax : nullptr;
+        const uint32_t nrow = rmz ? P + (merge || gu8 ? T : 0u) : 0u;
         L->last_T = T;
         L->last_P = P;
         L->last_S = S;
@@ -1659,7 +1678,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             hipLaunchKernelGGL(k_dispatch, dim3(1 + nsplit), dim3(1024), 0, ss, ids, P, E, tm, capf, counts, first, tiles,
                                pairs, inverse, S, K, xin, n, xh, xl, xs, (uint32_t)xord, (const float*)xstat, H, rmz,
                                nrow, ptiles, pcap);
-            if (hs && !merge && !dense8)
+            if (hs && !merge && !dn8)
                 hipLaunchKernelGGL(k_dense_tiles, dim3((scap + 63) / 64), dim3(64), 0, ss, T, scap, stiles);
         };
         L->stage_name[ST_DISPATCH] = "k_dispatch";
@@ -1685,7 +1704,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                   pairs, K, tiles, F, limit, act, so);
             }
             if (q8) split_act(ss, act, rmx, (uint64_t)(P + S), F, acth, actl);
-            if (dense8 && LL->pass.first) {
+            if (gu8 && LL->pass.first) {
                 launch_dense_q8(ss, true, xord, sgate.d, sup.d, sgate.stride, sup.stride, SF, H, xh, xl, T, limit, sact,
                                 xstat, rowmax + P);
             } else if (hs && !merge && LL->pass.first)
@@ -1712,7 +1731,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             else
                 launch_gemm<false>(ss, down.kind, dim3(H / 128, cap), down.d, nullptr, down.stride, 0, H, F, act,
                                    nullptr, K, tiles, H, 0.f, Y, so);
-            if (dense8 && LL->pass.first) {
+            if (dn8 && LL->pass.first) {
                 _Float16 *sh = acth + (uint64_t)P * F, *sl = actl + (uint64_t)P * F;
                 split_act(ss, sact, rowmax + P, T, SF, sh, sl);
                 launch_dense_q8(ss, false, A_NATURAL, sdown.d, nullptr, sdown.stride, 0ull, H, SF, sh, sl, T, 0.f, Ys,

@@ -43,6 +43,30 @@ def test_q8_shared_beside_other_formats(gpu, oracle, gk, dk):
     cached.destroy()
 
 
+@pytest.mark.parametrize("H,F,SF,T", [
+    (2048, 256, 64, 17), (2048, 256, 64, 200),     # one 64-column slab; down on the fp32 GEMM from 129 tokens
+    (2048, 256, 192, 70), (2048, 512, 320, 250),   # superblocks cut short; four tiles a block, the last in part (down)
+    (2048, 512, 320, 700),                         # four tiles a block (gate/up), down on the fp32 GEMM
+    (4096, 512, 512, 100), (4096, 512, 512, 450),  # wider x; four tiles a block (down; both)
+    (1024, 512, 512, 2048)])                       # the fp32 GEMM's rounds full: neither
+def test_q8_shared_shapes(gpu, oracle, H, F, SF, T):
+    """The shared expert's kernels at the edges of the rules that choose them. Each row
+    within 1e-5 of 64 bits: two 32-bit sums of at most 4096 products are 1.3e-6 off."""
+    K = 4 if T <= 64 else 1  # more than 64 pairs: not the decode kernels
+    spec = CF.make_layer(65, 0, H, 8, K, F, Q4_K, Q4_K, shared_ffn=SF, shared_gate_kind=Q8_0, shared_down_kind=Q8_0,
+                         shared_gated=True)
+    x = CF.inputs(65, T, H, seed=SF)
+    res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=3)
+    out, ids, _ = res(x)
+    st, ref, rids, _ = oracle.moe_forward(spec, x, oracle.F64)
+    assert st == 0 and np.array_equal(ids, rids)
+    err = np.linalg.norm(out - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= 1e-5, f"row {err.argmax()}: {err.max():.2e}"
+    assert np.array_equal(out, cached(x)[0])
+    res.destroy()
+    cached.destroy()
+
+
 @pytest.mark.parametrize("scale", [1e-12, 1e-4, 1e4, 1e12])
 def test_q8_any_activation_scale(gpu, oracle, scale):
     """No token-wise guess of the activations' size enters: the relative error
