@@ -67,7 +67,8 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 MFMA_F32_PEAK_TFLOPS = 157.3
-MFMA_F16_PEAK_TFLOPS = 2500.0  # dense fp16 MFMA, the datatype the f16 grouped GEMM issues
+MFMA_F16_PEAK_TFLOPS = 2500.0  # dense fp16 MFMA, the datatype the f16 grouped GEMMs issue
+F16_KERNELS = ("k_gemm_f16", "k_gemm_small")
 PROFILES = os.path.join(ROOT, "profiles")
 STAGE_ORDER = ("router", "route", "dispatch", "gate_up", "down", "combine")
 from ingot_amd.profile_summary import WORKLOADS as PROFILE_WORKLOADS  # noqa: E402
@@ -189,14 +190,14 @@ def kernel_roofline(bound, stage, stages, w, workload):
         peak, unit, algo = HBM_PEAK_GBS, "GB/s", {"algorithmic_bytes": w[stage]["bytes"]}
     else:
         achieved = w[stage]["flops"] / (us * 1e-6) / 1e12
-        f16 = kernel.startswith("k_gemm_f16")
+        f16 = kernel.startswith(F16_KERNELS)
         peak = MFMA_F16_PEAK_TFLOPS if f16 else MFMA_F32_PEAK_TFLOPS
         unit, algo = "TFLOP/s", {"algorithmic_flops": w[stage]["flops"]}
     traffic, src = measured_traffic(kernel, workload)
     r = {"bound": bound, "kernel": kernel, "stage": stage, "achieved": achieved, "peak": peak, "unit": unit,
          "frac": achieved / peak, "traffic": traffic, "traffic_source": src,
          "traffic_over_algorithmic_bytes": traffic / w[stage]["bytes"] if traffic else None, "kernel_us": us, **algo}
-    if bound == "mfma" and kernel.startswith("k_gemm_f16"):
+    if bound == "mfma" and kernel.startswith(F16_KERNELS):
         r["issued_f16_frac"] = 2.0 * achieved / MFMA_F16_PEAK_TFLOPS
         r["frac_vs_fp32_mfma_peak"] = achieved / MFMA_F32_PEAK_TFLOPS
         r["note"] = ("fp32-accurate products issued as two f16 MFMA products (A hi and lo) with fp32 "

@@ -1711,7 +1711,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                 launch_gemm<true>(ss, sgate.kind, dim3(SF / 64, scap), sgate.d, sup.d, sgate.stride, sup.stride, SF, H,
                                   xin, nullptr, 1, stiles, SF, limit, sact);
         };
-        L->stage_name[ST_GATEUP] = f16gu ? "k_gemm_f16<gate_up>" : "k_gemm<gate_up>";
+        L->stage_name[ST_GATEUP] = small ? "k_gemm_small<gate_up>" : f16gu ? "k_gemm_f16<gate_up>" : "k_gemm<gate_up>";
         L->stage[ST_DOWN] = [=](hipStream_t ss) {
             const uint32_t* so = LL->pass.slot_of;
             if (small)
@@ -1740,7 +1740,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                 launch_gemm<false>(ss, sdown.kind, dim3(H / 128, scap), sdown.d, nullptr, sdown.stride, 0, H, SF, sact,
                                    nullptr, 1, stiles, H, 0.f, Ys);
         };
-        L->stage_name[ST_DOWN] = f16 ? "k_gemm_f16<down>" : "k_gemm<down>";
+        L->stage_name[ST_DOWN] = small ? "k_gemm_small<down>" : f16 ? "k_gemm_f16<down>" : "k_gemm<down>";
         // The f16 down GEMM's rows of Y are in the act units of their token (Q8_0: true units).
         const float* yscale = f16 && !q8 ? xstat : nullptr;
         const uint32_t shared_scaled = merge ? 1u : 0u;

@@ -82,16 +82,18 @@ def _demangle(names):
 
 def stage_kernel(name: str) -> str:
     """The name bench.py and ingot_layer_stage_kernel use for a launched kernel:
-    k_gemm_f16<gate_up> / k_gemm_f16<down> (and k_gemm<...>) by their GATEUP
-    argument, k_router for both router kernels, otherwise the bare name."""
+    k_gemm_f16<gate_up> / k_gemm_f16<down> (and k_gemm_small<...>, k_gemm<...>, and
+    a shared expert's k_dense_q8<...> beside them) by their GATEUP argument,
+    k_router for both router kernels, otherwise the bare name."""
     m = re.search(r"(k_\w+?)(?:<([^>]*)>|I|E|\(|$)", name)
     if not m:
         return name
     base = m.group(1)
     args = [a.strip() for a in (m.group(2) or "").split(",")]
-    if base in ("k_gemm_f16", "k_gemm"):
-        if len(args) > 1:
-            gu = args[1] == "true"
+    if base in ("k_gemm_f16", "k_gemm_small", "k_gemm", "k_dense_q8"):
+        gates = [a for a in args if a in ("true", "false")]  # GATEUP is the first bool argument
+        if gates:
+            gu = gates[0] == "true"
         else:  # still mangled: ...ILi<kind>ELb<0|1>E...
             mm = re.search(r"Lb([01])E", name)
             gu = bool(mm and mm.group(1) == "1")

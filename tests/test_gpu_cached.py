@@ -63,7 +63,7 @@ def test_cached_layer_parity_and_counters(gpu, oracle, slots):
 @pytest.mark.parametrize("gk,dk", [(Q4_K, Q4_K), (Q5_K, Q5_K), (Q6_K, Q6_K), (Q4_K, Q6_K), (IQ2_XS, IQ2_XS),
                                    (IQ2_S, IQ4_XS), (IQ3_XXS, IQ4_NL), (IQ3_S, IQ3_S)])
 def test_cached_equals_resident_bit_for_bit(gpu, gk, dk):
-    """Prefill path, 160 pairs, merged shared expert. The resident layer's f16
+    """Prefill path, 160 pairs, merged shared expert. The resident layer's small-tile
     GEMMs read the tiled weight copies, the cached layer's read its slots in
     GGUF order; both decode the same operands and run the same products and
     combine, so the outputs are identical (which pins each tiled layout)."""
@@ -73,7 +73,7 @@ def test_cached_equals_resident_bit_for_bit(gpu, gk, dk):
     cached = MoeLayer(gpu, spec, cache_slots=5)
     o1, i1, w1 = res(x)
     o2, i2, w2 = cached(x)
-    assert res.stage_kernel(STAGE_DOWN) == "k_gemm_f16<down>"
+    assert res.stage_kernel(STAGE_DOWN) == "k_gemm_small<down>"
     assert np.array_equal(i1, i2) and np.array_equal(w1, w2)
     assert np.array_equal(o1, o2)
     assert cached.cache_stats()["misses"] == len(np.unique(i2))

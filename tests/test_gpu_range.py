@@ -74,12 +74,12 @@ def test_c1_shape_scaled_inputs(c1, oracle, scale):
 @pytest.mark.parametrize("scale", [1e-4, 3e3, 1e5])
 def test_c2_shape_scaled_inputs(c2, oracle, scale):
     """IQ2_XS layer with a gated Q8_0 shared expert: the v_dot2 decode GEMVs
-    (x and act split to f16 pairs) at 1 and 4 tokens, the f16 GEMM at 128."""
+    (x and act split to f16 pairs) at 1 and 4 tokens, the small-tile GEMM at 128."""
     spec, layer = c2
     for T in (1, 4, 128):
         x = CF.inputs(2, T, 2048, seed=7) * np.float32(scale)
         check_scaled(layer, spec, x, oracle, f"C2 shape x*{scale:g} T={T}")
-    assert layer.stage_kernel(STAGE_GATEUP) == "k_gemm_f16<gate_up>"
+    assert layer.stage_kernel(STAGE_GATEUP) == "k_gemm_small<gate_up>"
 
 
 def test_mixed_token_scales_one_batch(c1, oracle):

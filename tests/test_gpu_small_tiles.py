@@ -9,7 +9,8 @@ import numpy as np
 import pytest
 
 from ingot_amd import configs as CF
-from ingot_amd.moe import IQ2_S, IQ2_XS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q4_K, Q5_K, Q6_K, MoeLayer
+from ingot_amd.moe import (IQ2_S, IQ2_XS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q4_K, Q5_K, Q6_K, STAGE_DOWN, STAGE_GATEUP,
+                           MoeLayer)
 from util import check_layer
 
 pytestmark = pytest.mark.gpu
@@ -31,6 +32,18 @@ def routed_inputs(spec, loads, H, seed):
     return x
 
 
+def assert_rows_close(spec, x, out, oracle):
+    """Every row within 2^-15 of 64 bits. The split operands' products and the 32-bit
+    sums are good to about 2^-21 of the terms' size, and a row's terms cancel: the q and
+    min products of Q4_K and Q5_K (weights of +-2.5 sigma around a block's minimum) to
+    about 2^-2, a row whose g or u is small for its x to some 2^-4 of its terms in these
+    few hundred rows. A row whose lo parts were lost would be off by 2^-11 / sqrt(12), 2^-13."""
+    st, ref, _, _ = oracle.moe_forward(spec, x, oracle.F64)
+    assert st == 0
+    err = np.linalg.norm(out - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= 2.0 ** -15, f"row {err.argmax()}: {err.max():.2e}"
+
+
 @pytest.mark.parametrize("gk,dk,F", [(Q4_K, Q4_K, 256), (Q5_K, Q5_K, 768), (Q6_K, Q6_K, 256), (Q4_K, Q6_K, 768),
                                      (IQ2_XS, IQ2_XS, 512), (IQ2_S, IQ2_S, 512), (IQ3_XXS, IQ4_NL, 192),
                                      (IQ3_S, IQ3_S, 512), (IQ4_XS, IQ4_XS, 256), (IQ4_NL, IQ4_NL, 64)])
@@ -44,6 +57,9 @@ def test_tile_loads(gpu, oracle, gk, dk, F, shared):
         res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
         out, ids, _ = check_layer(res, spec, x, oracle, f"{gk}/{dk} F={F} shared={shared} {times}x loads")
         assert np.array_equal(np.bincount(ids.ravel(), minlength=E), loads)
+        assert_rows_close(spec, x, out, oracle)
+        gemm = "k_gemm_small" if times == 1 else "k_gemm_f16"
+        assert res.stage_kernel(STAGE_GATEUP) == f"{gemm}<gate_up>" and res.stage_kernel(STAGE_DOWN) == f"{gemm}<down>"
         assert np.array_equal(out, cached(x)[0]), "GGUF order against tiled copies"
         res.destroy()
         cached.destroy()

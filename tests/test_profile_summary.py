@@ -11,6 +11,11 @@ def test_stage_kernel_names():
     assert stage_kernel("void ingot::k_gemm_f16<12, true, 0, 128>(unsigned char const*)") == "k_gemm_f16<gate_up>"
     assert stage_kernel("void ingot::k_gemm_f16<18, false, 0, 64>(unsigned char const*)") == "k_gemm_f16<down>"
     assert stage_kernel("void ingot::k_gemm<8, true>(unsigned char const*)") == "k_gemm<gate_up>"
+    assert stage_kernel("void ingot::k_gemm_small<17, true, 2, true>(unsigned char const*)") == "k_gemm_small<gate_up>"
+    assert stage_kernel("void ingot::k_gemm_small<8, false, 0, true>(unsigned char const*)") == "k_gemm_small<down>"
+    assert stage_kernel("void ingot::k_dense_q8<true, 4, 1>(unsigned char const*)") == "k_dense_q8<gate_up>"
+    assert stage_kernel("void ingot::k_dense_q8<false, 0, 4>(unsigned char const*)") == "k_dense_q8<down>"
+    assert stage_kernel("_ZN5ingot10k_dense_q8ILb1ELi2ELi4EEEvPKhS2_mmjjPKDF16_S4_jfPfPKfPj") == "k_dense_q8<gate_up>"
     assert stage_kernel("void ingot::k_router_t<8, 16>(float const*)") == "k_router"
     assert stage_kernel("ingot::k_dec_gate_up2<12, 1, 3, 1, 2>(unsigned char const*)") == "k_dec_gate_up2"
     assert stage_kernel("ingot::k_combine(float const*)") == "k_combine"
