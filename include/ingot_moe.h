@@ -320,7 +320,9 @@ int ingot_layer_time_stage(ingot_layer* layer, uint32_t stage, uint32_t reps, fl
 /* The same over n layers (resident copies) replayed round-robin, so that
  * consecutive launches read weights at different addresses. */
 int ingot_layers_time_stage(ingot_layer* const* layers, uint32_t n, uint32_t stage, uint32_t reps, float* ms);
-/* Name of the HIP kernel that implements `stage` in the last forward. */
+/* Name of the HIP kernel that implements `stage` in the last forward (of two
+ * prefill GEMMs between which the dispatch chooses by its tile counts, the one
+ * that ran: synchronizes then; under capture the small-tile one). */
 const char* ingot_layer_stage_kernel(const ingot_layer* layer, uint32_t stage);
 /* The prefill dispatch of the last forward (synchronizes; INGOT_INVALID if that
  * forward ran the decode kernels, was a static forward, or a reserve has

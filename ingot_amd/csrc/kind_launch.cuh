@@ -152,7 +152,7 @@ bool launch_gemm_f16_k(hipStream_t s, int aord, bool tt128, bool tl, dim3 grid, 
     hipLaunchKernelGGL((k_gemm_f16<KIND, GATEUP, AO, TT, TLV>), grid, dim3(2 * TT), 0, s, a.w0, a.w1, a.ws0,     \
                        a.ws1, a.e_shared, a.stride0, a.stride1, a.rows_per_expert, a.kdim, a.ah, a.al, a.gs,     \
                        a.pairs, a.K, a.tiles, a.ldo, a.limit, a.out, a.out_h, a.out_l, a.out_gs, a.nblk,        \
-                       a.a_rows, a.xstat, a.rowmax, a.flags, a.slot_of)
+                       a.a_rows, a.xstat, a.rowmax, a.flags, a.slot_of, a.stiles)
 #define F16T(AO, TT)                    \
     do {                                \
         if (tl) F16L(AO, TT, true);     \

@@ -130,7 +130,8 @@ struct GemmF16Args {
     uint32_t* rowmax;
     uint32_t* flags;
     const uint32_t* slot_of;
-    uint32_t flat = 0;  // k_gemm_small: tile order
+    uint32_t flat = 0;                 // k_gemm_small: tile order
+    const uint32_t* stiles = nullptr;  // k_gemm_f16: k_gemm_small's list, and nothing to do unless it is empty
 };
 // The formats of the f16 grouped GEMM.
 #define INGOT_F16_KINDS(X) X(8) X(12) X(13) X(14) X(17) X(18) X(20) X(21) X(22) X(23)

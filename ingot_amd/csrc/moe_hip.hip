@@ -603,6 +603,7 @@ struct ingot_layer {
     // last_static: that forward used the shared static array
     uint32_t last_T = 0, last_P = 0, last_S = 0, last_cap = 0, last_tm = 0;
     bool last_prefill = false, last_static = false;
+    const uint32_t* last_pick = nullptr;  // the small-tile list (device) by which its dispatch chose the GEMM, or NULL
     Ws last;
     // flag word ctx->d_flags[slot]; seq: creation number on the context;
     // flag_status: what its kernels raised before the last flag check
@@ -697,14 +698,38 @@ static uint64_t carve(const ingot_layer* L, uint32_t T, void* base, Ws* out) {
 // 124.9 / 128.7.
 static const uint32_t GEMV_MAX_PAIRS = 64;
 
-// Batches of up to this many pairs per expert on average run k_gemm_small,
-// larger ones k_gemm_f16. Gate/up + down us, k_gemm_f16 against k_gemm_small:
-// 128 experts top-8 at 4 / 8 / 12 / 16 pairs per expert, Q4_K 104 / 108 / 110 /
-// 119 against 80 / 86 / 95 / 118, the Zipf-biased router 60 / 70 / - / 89 against
-// 41 / 58 / 73 / 90; IQ3_XXS / IQ4_NL at H = 4096, 4 / 8 / 16: 266 / 314 / 386
-// against 227 / 302 / 459; 512 IQ2_XS experts top-10 at 1.2 / 5 / 10: 269 / 328 /
-// 342 against 220 / 262 / 296.
-static const uint32_t SMALL_PAIRS_PER_EXPERT = 12;
+// Batches of up to this many half pairs per expert on average run k_gemm_small,
+// larger ones k_gemm_f16. Gate/up + down us, k_gemm_f16 against k_gemm_small, at 8 /
+// 12 / 14 or 16 pairs per expert and even routing: 128 experts top-8 of 768 x 2048
+// Q4_K 100 / 105 / 116 against 88 / 94 / 121, Q5_K 122 / 125 / 134 against 106 / 115 /
+// 137, Q6_K 137 / 141 / 146 against 129 / 137 / 151, Q8_0 160 / 165 / 173 against 140 /
+// 150 / 184, IQ4_XS 127 / 127 / 138 against 105 / 106 / 138, IQ4_NL 124 / 126 / 134
+// against 94 / 100 / 125; of 1024 x 2048 IQ3_XXS 119 / 123 / 123 against 107 / 114 / 125,
+// IQ3_S over IQ4_XS 150 / 150 / 163 against 129 / 135 / 165; 512 experts top-10 of 512 x
+// 2048 IQ2_XS 238 / 243 / 254 against 198 / 221 / 251, IQ2_S over IQ3_S 272 / 283 / 301
+// against 216 / 248 / 310, Q4_K 252 / 258 / - against 235 / 265 / -. IQ3_XXS over IQ4_NL at
+// 1408 x 4096, 10 / 11 / 12: 322 / 324 / 324 against 297 / 310 / 338. Q6_K gate/up, whose
+// k_gemm_f16 has 128-token tiles only, loses by more under skewed routing than it gains
+// under an even one: the Zipf-biased router at 4 / 8 / 12 pairs 53 / 64 / 82 against 56 /
+// 73 / 100 (even routing at 4: 131 against 114).
+static uint32_t small_half_pairs(uint32_t gate_kind) { return gate_kind == 14 ? 12u : gate_kind == 18 ? 23u : 24u; }
+
+// Where skewed routing could make many 16-pair tiles of few experts, each decoding its
+// weights again, the dispatch chooses by the tiles it counts: k_gemm_f16 if the 16-pair
+// tiles are more than 7 to 4 64-pair tiles (1.12 to 1 at 12 pairs per expert and even
+// routing) and give k_gemm_small more than 1536 gate/up blocks, 6 per CU (with fewer,
+// more blocks are worth more than fewer decodes). Both are then launched and the blocks
+// of one find nothing to do: 3 to 8 us in all, so it is done only above SKEW_WORK pairs x
+// F, below which no routing measured made k_gemm_small more than 7 % slower. Gate/up +
+// down us, k_gemm_f16 / k_gemm_small / the choice. 512 IQ2_XS experts of 512 x 2048
+// top-10, Zipf-biased router: 204 tokens (not above) 69 / 65 / 65, 409 tokens 91 / 104 /
+// 99, 614 114 / 141 / 119; all tokens to the same ten: 409 88 / 104 / 95; even: 409 223 /
+// 191 / 193. IQ3_XXS over IQ4_NL at 1408 x 4096, 128 experts top-8, Zipf: 64 tokens (not
+// above) 144 / 139 / 138, 128 203 / 219 / 220, 160 209 / 247 / 212; even: 128 315 / 275 /
+// 273. Q4_K over Q6_K, 256 experts of 768 x 2048 top-8, Zipf: 128 tokens (not above) 74 /
+// 58 / 58, 320 98 / 114 / 104; even: 320 215 / 204 / 207.
+static const uint64_t SKEW_WORK = 1228800;
+static const uint32_t SKEW_BLOCKS = 1536;
 
 // Whether a forward of T tokens takes the decode kernels (else routing,
 // dispatch and the grouped GEMMs). A cached layer reads the routing back to
@@ -784,6 +809,7 @@ static int reserve(ingot_layer* L, uint32_t T) {
         // the last forward's dispatch buffers and stage closures pointed into the freed block
         if (!L->last_static) {
             L->last_prefill = false;
+            L->last_pick = nullptr;
             for (auto& f : L->stage) f = nullptr;
         }
         HIP_TRY(ctx, hipMalloc(&ws, total));
@@ -1561,6 +1587,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         L->stage_name[ST_ROUTE] = "k_route";
     }
     L->last_prefill = !decode;
+    L->last_pick = nullptr;
     if (decode) {
         // router -> routed gate/up (block routing) [+ shared gate/up] -> down + combine
         const DevMatrix gate = L->gate, up = L->up, down = L->down, sgate = L->sgate, sup = L->sup, sdown = L->sdown;
@@ -1643,17 +1670,24 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         // The f16 GEMMs read the tiled copies where every matrix of the launch has one.
         const bool tlg = f16gu && gate.t && up.t && (!merge || (sgate.t && sup.t));
         const bool tld = f16 && down.t && (!merge || sdown.t);
-        // The small-tile GEMM up to SMALL_PAIRS_PER_EXPERT pairs per expert on average;
+        // The small-tile GEMM up to small_half_pairs half pairs per expert on average;
         // its tile list lies in w.act, which only an fp32 down GEMM and Q8_0 use (Q8_0:
         // in w.acts, the group sums that only Q4_K and Q5_K use).
         const uint32_t pcap = (P + TMS - 1) / TMS + E + (merge ? (T + TMS - 1) / TMS : 0u);
-        const bool small = f16 && P <= SMALL_PAIRS_PER_EXPERT * E && 16ull * pcap <= (q8 ? 4ull * P * (F / 32) : 4ull * P * F);
+        const bool small = f16 && 2ull * P <= (uint64_t)small_half_pairs(gate.kind) * E &&
+                           16ull * pcap <= (q8 ? 4ull * P * (F / 32) : 4ull * P * F);
         const uint32_t flat = P <= 8u * E ? 1u : 0u;
         uint32_t* const ptiles = small ? reinterpret_cast<uint32_t*>(q8 ? w.acts : w.act) : nullptr;
         const uint32_t tm = tt128 ? 2u * TM : TM;
         const uint8_t *g16 = tlg ? gate.t : gate.d, *u16 = tlg ? up.t : up.d, *d16 = tld ? down.t : down.d;
         const uint8_t *sg16 = tlg ? sgate.t : sgate.d, *su16 = tlg ? sup.t : sup.d, *sd16 = tld ? sdown.t : sdown.d;
         const uint32_t S = merge ? T : 0u, capf = cap + (merge ? scap : 0u), e_sh = merge ? E : 0xffffffffu;
+        const bool both = small && (uint64_t)P * F > SKEW_WORK;  // the dispatch chooses
+        const bool large = !small || both;
+        // k_gemm_f16's tiles if it is chosen: r rows of e experts make at most r / 16 + 15 e / 16
+        // tiles of 16, t >= e of 64, and 4 (r / 16 + 15 t / 16) > 7 t gives t < r / 13
+        const uint32_t cap16 = both ? std::min(capf, (P + S) / 13u + 2u) : capf;
+        const uint32_t pick = both ? SKEW_BLOCKS / (F / 64) : 0xffffffffu;
         _Float16 *xh = w.xh, *xl = w.xl, *acth = w.acth, *actl = w.actl;
         float *xs = w.xs, *acts = w.acts;
         // rows whose maxima the f16 gate/up raises (act split in the f16 GEMM's units)
@@ -1664,6 +1698,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         L->last_S = S;
         L->last_cap = capf;
         L->last_tm = tm;
+        L->last_pick = both ? ptiles : nullptr;
         auto split_act = [](hipStream_t ss, const float* a, const uint32_t* rm, uint64_t rows, uint32_t f, _Float16* h,
                             _Float16* l) {
             const uint64_t n = rows * f;
@@ -1677,7 +1712,7 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
             const uint32_t nsplit = (uint32_t)((n / 4 + 1023) / 1024);
             hipLaunchKernelGGL(k_dispatch, dim3(1 + nsplit), dim3(1024), 0, ss, ids, P, E, tm, capf, counts, first, tiles,
                                pairs, inverse, S, K, xin, n, xh, xl, xs, (uint32_t)xord, (const float*)xstat, H, rmz,
-                               nrow, ptiles, pcap);
+                               nrow, ptiles, pcap, pick);
             if (hs && !merge && !dn8)
                 hipLaunchKernelGGL(k_dense_tiles, dim3((scap + 63) / 64), dim3(64), 0, ss, T, scap, stiles);
         };
@@ -1692,14 +1727,15 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                         (const uint32_t*)pairs, K, (const uint32_t*)ptiles, F, limit, q8 ? act : (float*)nullptr,
                                         acth, actl, mins ? acts : nullptr, F / 64, T, (const float*)xstat, rmx, flags,
                                         so, flat);
-            } else if (f16gu) {
-                launch_gemm_f16<true>(ss, gate.kind, aord, tt128, tlg, dim3(8 * (F / 64) * ((capf + 7) / 8)), g16, u16,
+            }
+            if (large && f16gu) {
+                launch_gemm_f16<true>(ss, gate.kind, aord, tt128, tlg, dim3(8 * (F / 64) * ((cap16 + 7) / 8)), g16, u16,
                                       merge ? sg16 : nullptr, merge ? su16 : nullptr, e_sh, gate.stride, up.stride,
                                       F, H, (const _Float16*)xh, (const _Float16*)xl, (const float*)xs,
                                       (const uint32_t*)pairs, K, (const uint32_t*)tiles, F, limit,
                                       f16 && !q8 ? (float*)nullptr : act, acth, actl, mins ? acts : nullptr, F / 64, T,
-                                      (const float*)xstat, rmx, flags, so);
-            } else {
+                                      (const float*)xstat, rmx, flags, so, 0u, (const uint32_t*)(both ? ptiles : nullptr));
+            } else if (large) {
                 launch_gemm<true>(ss, gate.kind, dim3(F / 64, cap), gate.d, up.d, gate.stride, up.stride, F, H, xin,
                                   pairs, K, tiles, F, limit, act, so);
             }
@@ -1721,14 +1757,15 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
                                          (const float*)acts, (const uint32_t*)nullptr, K, (const uint32_t*)ptiles, H, 0.f,
                                          Y, (_Float16*)nullptr, (_Float16*)nullptr, (float*)nullptr, H / 128,
                                          (uint32_t)(P + S), (const float*)xstat, rmx, flags, so, flat);
-            else if (f16)
-                launch_gemm_f16<false>(ss, down.kind, A_NATURAL, tt128, tld, dim3(8 * (H / 128) * ((capf + 7) / 8)), d16,
+            if (large && f16)
+                launch_gemm_f16<false>(ss, down.kind, A_NATURAL, tt128, tld, dim3(8 * (H / 128) * ((cap16 + 7) / 8)), d16,
                                        (const uint8_t*)nullptr, merge ? sd16 : nullptr, (const uint8_t*)nullptr, e_sh,
                                        down.stride, 0ull, H, F, (const _Float16*)acth, (const _Float16*)actl,
                                        (const float*)acts, (const uint32_t*)nullptr, K, (const uint32_t*)tiles, H, 0.f,
                                        Y, (_Float16*)nullptr, (_Float16*)nullptr, (float*)nullptr, H / 128,
-                                       (uint32_t)(P + S), (const float*)xstat, rmx, flags, so);
-            else
+                                       (uint32_t)(P + S), (const float*)xstat, rmx, flags, so, 0u,
+                                       (const uint32_t*)(both ? ptiles : nullptr));
+            else if (large)
                 launch_gemm<false>(ss, down.kind, dim3(H / 128, cap), down.d, nullptr, down.stride, 0, H, F, act,
                                    nullptr, K, tiles, H, 0.f, Y, so);
             if (dn8 && LL->pass.first) {
@@ -1856,6 +1893,15 @@ int ingot_layer_time_stage(ingot_layer* L, uint32_t stage, uint32_t reps, float*
 
 const char* ingot_layer_stage_kernel(const ingot_layer* L, uint32_t stage) {
     if (!L || stage >= ST_N || !L->stage[stage]) return "";
+    if (L->last_pick && (stage == ST_GATEUP || stage == ST_DOWN)) {
+        // The dispatch's choice: the small-tile list's count.
+        uint32_t n = 1;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(L->ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone &&
+            hipStreamSynchronize(L->ctx->stream) == hipSuccess)
+            (void)hipMemcpy(&n, L->last_pick + 3, 4, hipMemcpyDeviceToHost);
+        if (n == 0) return stage == ST_GATEUP ? "k_gemm_f16<gate_up>" : "k_gemm_f16<down>";
+    }
     return L->stage_name[stage];
 }
 

@@ -1603,7 +1603,7 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
                                                    float* __restrict__ xs, uint32_t xorder,
                                                    const float* __restrict__ xstat, uint32_t H,
                                                    uint32_t* __restrict__ rowmax, uint32_t nrow,
-                                                   uint32_t* __restrict__ stiles, uint32_t scap) {
+                                                   uint32_t* __restrict__ stiles, uint32_t scap, uint32_t pick) {
     if (blockIdx.x > 0) {
         split_f16_part(x, xn, xh, xl, xs, xorder, (uint64_t)(blockIdx.x - 1u) * blockDim.x + threadIdx.x, xstat, H);
         return;
@@ -1646,7 +1646,9 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
     }
     const uint32_t nfull = n / TM, rem = n - nfull * TM;
     // stiles != NULL: also the tile list of the small-tile GEMM (tiles of TMS
-    // pairs, the same order); its counts ride in the upper halves of the scans.
+    // pairs, the same order); its counts ride in the upper halves of the scans. It
+    // stays empty when it has more than `pick` tiles and more than 7 of them to 4
+    // TM-pair tiles: k_gemm_f16 runs then.
     const uint32_t sfull = n / TMS, srem = n - sfull * TMS, half = stiles ? 0xffffu : 0xffffffffu;
     const uint32_t f = block_exclusive_scan_1024(n, wsum, &tot[0]);
     __syncthreads();
@@ -1677,12 +1679,14 @@ __global__ __launch_bounds__(1024) void k_dispatch(const uint32_t* __restrict__ 
     if (stiles && tid < TMS - 1u) sbin[TMS - 1u - tid] = ssh + sfull_all + (before >> 16);
     __syncthreads();
     if (stiles) {
-        const uint32_t nst = min(ssh + sfull_all + (tot[2] >> 16), scap);
+        const uint32_t nst_all = ssh + sfull_all + (tot[2] >> 16), nt64 = nsh + nfull_all + nt_all;
+        const bool take = nst_all <= pick || 4u * nst_all <= 7u * nt64;
+        const uint32_t nst = take ? min(nst_all, scap) : 0u;
         auto put = [&](uint32_t t, uint32_t e, uint32_t q, uint32_t m) {
             if (t < scap) *reinterpret_cast<uint4*>(stiles + 4u * t) = make_uint4(e, q, m, nst);
         };
-        for (uint32_t j = tid; j < ssh; j += 1024u) put(j, E, P + j * TMS, min(TMS, S - j * TMS));
-        if (tid < E) {
+        for (uint32_t j = tid; take && j < ssh; j += 1024u) put(j, E, P + j * TMS, min(TMS, S - j * TMS));
+        if (take && tid < E) {
             for (uint32_t k = 0; k < sfull; ++k) put(ssh + (t0s >> 16) + k, tid, f + k * TMS, TMS);
             if (srem) put(atomicAdd(&sbin[srem], 1u), tid, f + sfull * TMS, srem);
         }
@@ -2774,7 +2778,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     const uint32_t* __restrict__ pairs, uint32_t K, const uint32_t* __restrict__ tiles, uint32_t ldo, float limit,
     float* __restrict__ out, _Float16* __restrict__ out_h, _Float16* __restrict__ out_l, float* __restrict__ out_gs,
     uint32_t nblk, uint32_t a_rows, const float* __restrict__ xstat, uint32_t* __restrict__ rowmax,
-    uint32_t* __restrict__ flags, const uint32_t* __restrict__ slot_of) {
+    uint32_t* __restrict__ flags, const uint32_t* __restrict__ slot_of, const uint32_t* __restrict__ stiles) {
     static_assert(KIND == 8 || KIND == 12 || KIND == 13 || KIND == 14 || KIND == 17 || KIND == 18 || KIND == 20 || KIND == 21 ||
                       KIND == 22 || KIND == 23,
                   "f16 GEMM formats: Q8_0, Q4_K, Q5_K, Q6_K, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_NL, IQ4_XS");
@@ -2807,6 +2811,7 @@ __global__ __launch_bounds__(TT * 2) __attribute__((amdgpu_waves_per_eu(2))) voi
     // measured block times: XCD spans 62-85 us against 70-76 us snaked;
     // measured: C1 gate/up about 1.4 us shorter, C3 gate/up 176-178 to
     // 169-170 us, C3 down 114-116 to 111-113).
+    if (stiles != nullptr && stiles[3] != 0u) return;  // the dispatch chose the small-tile GEMM
     const uint32_t nt = tiles[3], slot = blockIdx.x >> 3, ti = slot / nblk, xcd = blockIdx.x & 7u;
     const uint32_t t = ti * 8u + ((ti & 1u) ? 7u - xcd : xcd);
     if (t >= nt) return;

@@ -2,14 +2,15 @@
 expert loads at the edges of the small-tile GEMM's operands (8 pairs packed hi
 and lo in one operand, 16 pairs per tile) and just past them, empty experts, a
 K that ends inside an A chunk, merged shared tiles; and the same loads doubled,
-past the rule that selects the small tiles (12 pairs per expert). Against the
-oracle, to the repository's bar; and GGUF-order weights (a cached layer) bit for
+past the rule that selects the small tiles (11 to 12 pairs per expert). Against the
+oracle, to the repository's bar, and every row closely; the dispatch's choice between
+the two kernels on both sides of its tile counts; and GGUF-order weights (a cached layer) bit for
 bit against the tiled copies (a resident one)."""
 import numpy as np
 import pytest
 
 from ingot_amd import configs as CF
-from ingot_amd.moe import (IQ2_S, IQ2_XS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q4_K, Q5_K, Q6_K, STAGE_DOWN, STAGE_GATEUP,
+from ingot_amd.moe import (IQ2_S, IQ2_XS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q4_K, Q5_K, Q6_K, Q8_0, STAGE_DOWN, STAGE_GATEUP,
                            MoeLayer)
 from util import check_layer
 
@@ -49,10 +50,11 @@ def assert_rows_close(spec, x, out, oracle):
                                      (IQ3_S, IQ3_S, 512), (IQ4_XS, IQ4_XS, 256), (IQ4_NL, IQ4_NL, 64)])
 @pytest.mark.parametrize("shared", [False, True])
 def test_tile_loads(gpu, oracle, gk, dk, F, shared):
-    H, E = 1024, len(LOADS)
+    base = LOADS + [0] * (16 if gk == Q6_K else 0)  # Q6_K gate/up: up to 6 pairs per expert
+    H, E = 1024, len(base)
     spec = CF.make_layer(61, 0, H, E, 1, F, gk, dk, shared_ffn=F if shared else 0)
     for times in (1, 2):  # small tiles; past the rule
-        loads = [times * v for v in LOADS]
+        loads = [times * v for v in base]
         x = routed_inputs(spec, loads, H, 61 + times)
         res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=5)
         out, ids, _ = check_layer(res, spec, x, oracle, f"{gk}/{dk} F={F} shared={shared} {times}x loads")
@@ -63,3 +65,30 @@ def test_tile_loads(gpu, oracle, gk, dk, F, shared):
         assert np.array_equal(out, cached(x)[0]), "GGUF order against tiled copies"
         res.destroy()
         cached.destroy()
+
+
+# 64 experts of 1792 (28 gate/up blocks a tile): the dispatch chooses from 686 pairs on, k_gemm_f16 above
+# 54 tiles of 16 pairs if they are more than 7 to 4 64-pair tiles.
+@pytest.mark.parametrize("loads,shared,f16", [
+    ([12] * 64, False, False),
+    ([224, 224, 240] + [1] * 11, False, False), ([224, 224, 240] + [1] * 12, False, True),  # 54 tiles; 55
+    ([48] * 12 + [6] * 20, False, False), ([48] * 13 + [4] * 18, False, True),  # 56 to 32; 57 to 31
+    ([250, 250, 240] + [1] * 27, True, True)])
+@pytest.mark.parametrize("gk,dk", [(Q4_K, Q6_K), (Q8_0, Q8_0)])
+def test_dispatch_chooses_by_tiles(gpu, oracle, gk, dk, loads, shared, f16):
+    H, E, F = 1024, 64, 1792
+    spec = CF.make_layer(66, 0, H, 4, 1, F, gk, dk, shared_ffn=F if shared else 0)
+    spec.experts = E
+    for m in ("gate", "up", "down"):
+        setattr(spec, m, getattr(spec, m).select([(5 * e) % 4 for e in range(E)]))
+    loads = loads + [0] * (E - len(loads))
+    x = routed_inputs(spec, loads, H, 66)
+    res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=40)
+    out, ids, _ = res(x)
+    assert np.array_equal(np.bincount(ids.ravel(), minlength=E), loads)
+    gemm = "k_gemm_f16" if f16 else "k_gemm_small"
+    assert res.stage_kernel(STAGE_GATEUP) == f"{gemm}<gate_up>" and res.stage_kernel(STAGE_DOWN) == f"{gemm}<down>"
+    assert_rows_close(spec, x, out, oracle)
+    assert np.array_equal(out, cached(x)[0])
+    res.destroy()
+    cached.destroy()
