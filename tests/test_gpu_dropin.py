@@ -8,7 +8,7 @@ import pytest
 
 from ingot_amd import configs as CF
 from ingot_amd.moe import (BF16, F16, F32, IQ1_M, IQ2_S, IQ2_XS, IQ2_XXS, IQ3_S, IQ3_XXS, IQ4_NL, IQ4_XS, Q2_0, Q2_K,
-                           Q4_0, Q4_K, Q5_K, Q6_K, Q8_0, ROUTE_SIGMOID, ROUTE_SOFTMAX, InvalidData, Matrix)
+                           Q4_0, Q4_K, Q5_K, Q6_K, Q8_0, ROUTE_SIGMOID, ROUTE_SOFTMAX, Gpu, InvalidData, Matrix)
 from util import assert_close
 
 pytestmark = pytest.mark.gpu
@@ -174,6 +174,34 @@ def test_moe_dropin_matches_oracle(gpu, oracle):
     sgate = Matrix(gvec.view(np.uint8).copy(), 2048, 1, 1, F32, 4 * 2048)
     out = gpu.moe(routed, list(spec.shared), sgate, x[0], w[0])
     assert_close(out, ref[0], "Gpu::moe")
+
+
+def test_moe_dropin_reuses_and_grows_its_block(gpu, oracle):
+    """One context, calls of several sizes: the kept device block is grown, reused by a
+    smaller call and passed over by one of more than 64 MiB, and given back with the
+    context."""
+    sizes = [(256, True), (768, False), (3072, True), (256, False), (768, True)]  # 7 to 23 MB; 3072: 88 MB
+    calls = []
+    for i, (F, shared) in enumerate(sizes):
+        spec = CF.make_layer(42, i, 2048, 8, 8, F, Q4_K, Q4_K, shared_ffn=256 if shared else 0, shared_gated=shared)
+        x = CF.inputs(42, 1, 2048, seed=i)
+        st, ref, ids, w = oracle.moe_forward(spec, x, oracle.F64)
+        assert st == 0
+        sel = list(ids[0])
+        sgate = None
+        if shared:
+            sgate = Matrix(spec.shared_gate_vec.astype(np.float32).view(np.uint8).copy(), 2048, 1, 1, F32, 4 * 2048)
+        calls.append(([spec.gate.select(sel), spec.up.select(sel), spec.down.select(sel)],
+                      list(spec.shared) if shared else None, sgate, x[0], w[0], ref[0]))
+    gpu.moe(*calls[0][:5])  # code objects loaded
+    own = Gpu(0)
+    free0, _ = gpu.mem_info()
+    for (F, shared), (routed, sh, sgate, x, w, ref) in zip(sizes, calls):
+        assert_close(own.moe(routed, sh, sgate, x, w), ref, f"Gpu::moe F={F} shared={shared}")
+        free, _ = gpu.mem_info()
+        assert free0 - free <= 66 << 20, f"F={F}: {free0 - free} bytes kept"  # 64 MiB and a page of 2 MiB
+    own.close()
+    assert gpu.mem_info()[0] >= free0
 
 
 def test_moe_dropin_errors(gpu):
