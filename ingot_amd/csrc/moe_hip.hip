@@ -212,17 +212,25 @@ bool tiled_kind(const DevMatrix& m) {
     return cols_ok && m.rows % 16 == 0;
 }
 
+// Room for m's tiled copy, or NULL: the copy is optional, and without it the GEMM keeps
+// reading GGUF order. Q8_0, the largest format, leaves a sixteenth of the card to the
+// workspaces of later layers and the caller, whose allocations fail a call and not just
+// a copy.
+uint8_t* alloc_tiled(const DevMatrix& m) {
+    void* t = nullptr;
+    size_t avail = 0, total = 0;
+    if (m.kind == 8 && (hipMemGetInfo(&avail, &total) != hipSuccess || avail < m.nbytes + total / 16)) return nullptr;
+    if (hipMalloc(&t, m.nbytes) == hipSuccess) return static_cast<uint8_t*>(t);
+    (void)hipGetLastError();
+    return nullptr;
+}
+
 // m->t = m->d in the tiled layout (resident layers, at the first reserve of a
 // batch that takes the prefill path; the decode kernels and the fp32 GEMM
 // keep reading m->d).
 int make_tiled(ingot_ctx* ctx, DevMatrix* m) {
     if (!m->d || m->t || !tiled_kind(*m)) return INGOT_OK;
-    // The copy is optional: without room for it the GEMM keeps reading GGUF order.
-    if (hipMalloc(reinterpret_cast<void**>(&m->t), m->nbytes) != hipSuccess) {
-        (void)hipGetLastError();
-        m->t = nullptr;
-        return INGOT_OK;
-    }
+    if (!(m->t = alloc_tiled(*m))) return INGOT_OK;
     const uint64_t blocks = std::min<uint64_t>((m->nbytes + 255) / 256, 1u << 20);
     hipLaunchKernelGGL(k_tile_weights, dim3((uint32_t)blocks), dim3(256), 0, ctx->stream, m->d, m->t, m->nbytes,
                        m->kind, m->stride);
@@ -1385,7 +1393,11 @@ int ingot_layer_clone(const ingot_layer* src, ingot_layer** out) {
         *dm[i] = *sm[i];
         dm[i]->d = dm[i]->t = nullptr;
         st = dup(sm[i]->d, sm[i]->nbytes, (void**)&dm[i]->d);
-        if (st == INGOT_OK) st = dup(sm[i]->t, sm[i]->nbytes, (void**)&dm[i]->t);
+    }
+    for (int i = 0; i < 6 && st == INGOT_OK; ++i) {
+        if (!sm[i]->t || !(dm[i]->t = alloc_tiled(*sm[i]))) continue;
+        const hipError_t e = hipMemcpy(dm[i]->t, sm[i]->t, sm[i]->nbytes, hipMemcpyDeviceToDevice);
+        if (e != hipSuccess) st = fail(ctx, INGOT_DEVICE, std::string("hipMemcpy: ") + hipGetErrorString(e));
     }
     if (st == INGOT_OK) st = attach(ctx, L);
     if (st != INGOT_OK) {

@@ -66,6 +66,34 @@ def test_q8_shared_shapes(gpu, oracle, H, F, SF, T):
     cached.destroy()
 
 
+def test_q8_copies_leave_room(gpu):
+    """The second copies of a Q8_0 layer's weights are not made on a nearly full card (a
+    sixteenth of it is left), and the layer computes the same without them."""
+    spec = CF.make_layer(67, 0, 1024, 32, 4, 512, Q8_0, Q8_0)
+    x = CF.inputs(67, 70, 1024)
+    full, roomy = MoeLayer(gpu, spec), MoeLayer(gpu, spec)
+    bytes_ = full.weight_bytes()
+    roomy.reserve(70)
+    total = gpu.mem_info()[1]
+    fill = []
+    for _ in range(64):  # nothing touches it
+        left = gpu.mem_info()[0] - total // 16 - (8 << 20)
+        if left < 2 << 20:
+            break
+        fill.append(gpu.buffer(min(left, 32 << 30)))
+    out = full(x)[0]
+    kept, avail = full.weight_bytes(), gpu.mem_info()[0]
+    clone = roomy.clone()  # its weights, without their copies
+    cloned = clone.weight_bytes()
+    for b in fill:
+        b.free()
+    assert kept == bytes_ and avail > total // 16 - (16 << 20)  # less the workspace
+    assert cloned == bytes_ and np.array_equal(out, clone(x)[0])
+    assert np.array_equal(out, roomy(x)[0]) and roomy.weight_bytes() > 2 * bytes_ - (1 << 20)
+    for layer in (full, roomy, clone):
+        layer.destroy()
+
+
 @pytest.mark.parametrize("scale", [1e-12, 1e-4, 1e4, 1e12])
 def test_q8_any_activation_scale(gpu, oracle, scale):
     """No token-wise guess of the activations' size enters: the relative error
