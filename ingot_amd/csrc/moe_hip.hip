@@ -755,6 +755,8 @@ static bool takes_decode(const ingot_layer* L, uint32_t T) {
 // The f16 GEMM addresses its A operands (x split: T rows of H; act split: P + T
 // rows of F) and their group sums with 32-bit byte offsets.
 static bool f16_gemm_fits(uint64_t kdim, uint64_t rows) { return 2ull * kdim * rows < (1ull << 32); }
+// And an expert's weights (the fp32 GEMM: 64-bit addresses).
+static bool f16_weights_fit(const DevMatrix& m) { return m.rows * m.stride < (1ull << 32); }
 
 // Which prefill GEMMs a batch of T tokens runs. f16gu: gate/up on the f16 GEMM
 // (both projections' formats allow it, or only gate/up's, which then writes
@@ -775,8 +777,9 @@ static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
     // its row maxima (k_split_act), the other formats' in units of the token.
     const bool q8 = L->gate.kind == 8;
     p.f16gu = L->gemm_mode == INGOT_GEMM_AUTO && f16_gemm_kind(L->gate.kind, L->H, true) && f16_gemm_fits(L->H, T) &&
-              f16_gemm_fits(L->F, PS) && (!q8 || L->down.kind == 8);
-    p.f16 = p.f16gu && f16_gemm_kind(L->down.kind, L->F, false) && (q8 || L->down.kind != 8);
+              f16_gemm_fits(L->F, PS) && f16_weights_fit(L->gate) && f16_weights_fit(L->up) &&
+              (!q8 || (L->down.kind == 8 && f16_weights_fit(L->down)));
+    p.f16 = p.f16gu && f16_weights_fit(L->down) && f16_gemm_kind(L->down.kind, L->F, false) && (q8 || L->down.kind != 8);
     p.merge = p.f16 && L->has_shared && L->SF == L->F && L->sgate.kind == L->gate.kind &&
               L->sup.kind == L->up.kind && L->sdown.kind == L->down.kind && L->sgate.stride == L->gate.stride &&
               L->sup.stride == L->up.stride && L->sdown.stride == L->down.stride;
@@ -795,7 +798,7 @@ static PrefillPlan prefill_plan(const ingot_layer* L, uint32_t T) {
     // The down product takes it after the gate/up product only (for the row maxima), so
     // a nearly full gate/up round is given up where the down product gains more.
     if (p.f16gu && L->has_shared && !p.merge && L->sgate.kind == 8 && L->sdown.kind == 8 && L->SF <= L->F &&
-        a_order(L->gate.kind) != A_IQ4NL) {
+        f16_weights_fit(L->sgate) && f16_weights_fit(L->sdown) && a_order(L->gate.kind) != A_IQ4NL) {
         const uint64_t tt = (T + TM - 1) / TM, gu = tt * (L->SF / 64), dn = tt * (L->H / 128);
         p.dn8 = dn <= 256 ? 2 * dn <= L->SF : L->SF >= 512 && !fills(dn, 80);
         p.gu8 = !fills(gu, p.dn8 ? 95 : 80);

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from ingot_amd import configs as CF
-from ingot_amd.moe import IQ2_XS, IQ4_NL, Q4_K, Q6_K, Q8_0, STAGE_DOWN, STAGE_GATEUP, MoeLayer
+from ingot_amd.moe import IQ2_XS, IQ4_NL, Q4_K, Q6_K, Q8_0, STAGE_DOWN, STAGE_GATEUP, LayerSpec, Matrix, MoeLayer
 from test_gpu_small_tiles import LOADS, assert_rows_close, routed_inputs
 from util import check_layer
 
@@ -64,6 +64,32 @@ def test_q8_shared_shapes(gpu, oracle, H, F, SF, T):
     assert np.array_equal(out, cached(x)[0])
     res.destroy()
     cached.destroy()
+
+
+def test_q8_expert_of_4_gib(gpu):
+    """Matrices whose bytes do not fit the f16 GEMM's 32-bit offsets stay on the fp32 GEMM:
+    an expert with only its last 64 columns of act in use, at 4 GiB into gate and up."""
+    H, F = 1024, 1 << 22
+    gate, up, down = (np.zeros(n, np.uint8) for n in (F * 1088, F * 1088, H * (F // 32 * 34)))
+    rng = np.random.default_rng(68)
+    scale = np.frombuffer(np.float16(0.002).tobytes(), np.uint8)
+    values = []
+    for m, rows, blocks in ((gate, slice(F - 64, F), slice(0, 32)), (up, slice(F - 64, F), slice(0, 32)),
+                            (down, slice(0, H), slice(F // 32 - 2, F // 32))):
+        b = m.reshape(-1, H // 32 if m is not down else F // 32, 34)[rows, blocks]
+        b[..., :2] = scale
+        b[..., 2:] = rng.integers(0, 256, b.shape[:2] + (32,))
+        values.append(b[..., 2:].view(np.int8).reshape(len(b), -1) * np.float64(np.float16(0.002)))
+    mats = [Matrix(gate, H, F, 1, Q8_0, 1088), Matrix(up, H, F, 1, Q8_0, 1088), Matrix(down, F, H, 1, Q8_0, F // 32 * 34)]
+    x = CF.inputs(68, 3, H)
+    layer = MoeLayer(gpu, LayerSpec(hidden=H, experts=1, top_k=1, router=np.zeros((1, H), np.float32), gate=mats[0],
+                                    up=mats[1], down=mats[2]))
+    out = layer(x)[0]
+    g, u = x @ values[0].T, x @ values[1].T
+    ref = (g / (1.0 + np.exp(-g)) * u) @ values[2].T
+    assert np.linalg.norm(out - ref) <= 1e-5 * np.linalg.norm(ref)  # two 32-bit sums of at most 1024 products
+    assert layer.stage_kernel(STAGE_GATEUP) == "k_gemm<gate_up>"
+    layer.destroy()
 
 
 def test_q8_copies_leave_room(gpu):
