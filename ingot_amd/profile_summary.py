@@ -220,8 +220,10 @@ LDS_PASS = ("SQ_WAVE_CYCLES SQ_WAIT_ANY SQ_WAIT_INST_ANY SQ_ACTIVE_INST_VALU SQ_
             "SQ_ACTIVE_INST_VMEM SQ_LDS_BANK_CONFLICT SQ_WAIT_INST_LDS")
 LDS_FILES = {
     "gemm_lds_conflicts_c1_c3.md": (
-        "LDS bank conflicts and wave stalls of the f16 GEMM: C1 prefill 512 and C3 T=64",
-        (("c1", "C1 prefill 512"), ("c3", "C3 T=64")), "k_gemm_f16"),
+        "LDS bank conflicts and wave stalls of the prefill GEMMs: C1 prefill 512, C3 T=64 and the IQ2_S/IQ3_S mix at "
+        "prefill 512",
+        (("c1", "C1 prefill 512"), ("c3", "C3 T=64"), ("mixiqp", "IQ2_S/IQ3_S prefill 512")),
+        ("k_gemm", "k_dense_q8")),
     "decode_waits_c0_c2.md": (
         "Wave stalls of the decode kernels: C0 decode b=1 and C2 decode b=1",
         (("c0", "C0 b=1"), ("c2b1", "C2 b=1")), "k_"),
