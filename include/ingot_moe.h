@@ -147,7 +147,9 @@ int ingot_dequant(ingot_ctx* ctx, const ingot_matrix* m, float* out);
 /* Gpu::moe: routed[3] = gate, up, down holding the K selected experts
  * (count = K, expert k uses weights[k]); shared[3] and shared_gate (a
  * [cols = H, rows = 1] matrix) may be NULL for a layer without a shared
- * expert; out[H] = sum_k w_k E_k(x) + sigmoid(shared_gate . x) S(x). */
+ * expert; out[H] = sum_k w_k E_k(x) + sigmoid(shared_gate . x) S(x). The
+ * context keeps the call's device memory, up to 64 MiB, for the next one until
+ * it is destroyed; a call that needs more allocates and frees its own. */
 int ingot_moe(ingot_ctx* ctx, const ingot_matrix routed[3], const ingot_matrix* shared,
               const ingot_matrix* shared_gate, const float* x, const float* weights, uint32_t K,
               float* out);
@@ -206,7 +208,10 @@ typedef struct ingot_layer_desc {
  * copy at the first ingot_layer_reserve (or forward) of a batch that takes
  * the prefill path: the same bytes reordered so that each of that GEMM's
  * weight loads reads one contiguous span. It doubles those matrices' device
- * memory; a layer that only decodes never makes it. */
+ * memory; a layer that only decodes never makes it, nor one set to
+ * INGOT_GEMM_FP32 before. Without room for a copy the GEMM reads the matrix as
+ * it is; a Q8_0 matrix is copied only while a sixteenth of the card stays free
+ * after it. */
 int ingot_layer_create(ingot_ctx* ctx, const ingot_layer_desc* desc, ingot_layer** out);
 /* A second resident copy of the same weights at new device addresses (not for
  * cached layers). */
@@ -290,9 +295,13 @@ int ingot_layer_forward_add(ingot_layer* layer, const float* d_x, const float* d
  * ingot_ctx_check_device_flags reports as INGOT_RANGE, and its outputs must
  * be recomputed with INGOT_GEMM_FP32. Layers whose gate, up and down are all
  * Q8_0 run on it too (B the int8 value, f16 hi + lo scaled by each activation
- * row's own maximum, so without a range); beside another format a Q8_0
- * projection keeps the fp32 GEMM.
- * INGOT_GEMM_FP32: always the fp32 MFMA GEMM. */
+ * row's own maximum, so without a range), and so may a Q8_0 shared expert
+ * (gate, up and down) beside routed experts of another such format, where the
+ * fp32 GEMM would leave CUs idle; a routed Q8_0 projection beside another
+ * format keeps the fp32 GEMM. A split operand holds 22 to 23 bits of each value
+ * down to 2^-13 of its row's largest, below that an absolute step of 2^-35 of
+ * the largest; products are exact and sums are fp32.
+ * INGOT_GEMM_FP32: always the fp32 MFMA GEMM, for the shared expert too. */
 enum ingot_gemm_mode { INGOT_GEMM_AUTO = 0, INGOT_GEMM_FP32 = 1 };
 int ingot_layer_set_gemm_mode(ingot_layer* layer, uint32_t mode);
 /* Device bytes held by the layer's weights (with the reordered copies). */

@@ -7,9 +7,11 @@
 // there is stalls: 2 waves per SIMD, a barrier and an A DMA per 64 columns.
 // Here
 //   * a block is 4 waves over 64 act columns (gate/up: 16 gate and the same 16
-//     up rows per wave) or 128 down rows (32 per wave), at most 128 VGPRs, so
-//     four blocks fit a CU and each wave keeps four slabs of its weights in
-//     flight;
+//     up rows per wave) or 128 down rows (32 per wave). From the tiled copies
+//     four blocks fit a CU (at most 128 VGPRs, 33 to 40 KB of LDS), three for
+//     Q8_0 and Q6_K (up to 142 VGPRs) and IQ2_S (45 KB); in GGUF order three of
+//     those that need more than 128 VGPRs, two of Q6_K. Each wave keeps four
+//     slabs of its weights in flight;
 //   * A is staged in LDS in chunks of 16 KB (two buffers, one barrier per
 //     chunk): tiles of at most 8 pairs hold their hi rows in MFMA rows 0..7 and
 //     the lo rows in rows 8..15 of ONE operand (512 columns per chunk), so each
@@ -20,9 +22,10 @@
 //     unit (one fma per value), which needs no reciprocal of the next unit.
 // Gate/up + down, k_gemm_f16 against this kernel: a Qwen3-30B-A3B-shaped layer
 // (Q4_K / Q6_K) at 32 tokens 109 -> 88 us (4.0 TB/s of weights in gate/up), the
-// GLM-shaped IQ3_XXS / IQ4_NL layer at 64 tokens 266 -> 227 us. The vector ALU is
-// then about half busy with the decode (Q4_K); the IQ formats are bound by their
-// codebook reads from LDS.
+// GLM-shaped IQ3_XXS / IQ4_NL layer at 64 tokens 266 -> 227 us. By counters, gate/up
+// of the first then issues VALU instructions in 40 % of its SIMD cycles and its waves
+// spend 47 % of theirs waiting for loads and the barrier; in the second's LDS bank
+// conflicts, nearly all of the codebook reads, take 43 % of a CU's cycles.
 #pragma once
 #include "moe_kernels.cuh"
 

@@ -1659,12 +1659,12 @@ static int layer_forward(ingot_layer* L, const Ws& w, const float* d_x, const fl
         float *act = w.act, *sact = w.sact, *Y = w.Y, *Ys = w.Y + (uint64_t)P * H, limit = L->limit;
         const float* wts = w.wts;
         bool hs = L->has_shared;
-        // The f16 GEMM runs when both projections' formats allow it; the shared
-        // expert then joins the same launches (as tile expert E over rows
-        // P..P+T-1) when it has the routed experts' formats and width, and
-        // otherwise runs on the fp32 GEMM beside them. When only gate/up's
-        // format allows it (a Q4_K_M layer's Q6_K down), gate/up runs on the
-        // f16 GEMM writing fp32 act and the down projection on the fp32 GEMM,
+        // The f16 GEMMs run when both projections' formats allow it (Q8_0: all of gate,
+        // up and down); the shared expert then joins the same launches (as tile expert
+        // E over rows P..P+T-1) when it has the routed experts' formats and width. A
+        // Q8_0 one beside other formats may run on k_dense_q8, and any other on the
+        // fp32 GEMM. When only gate/up's format allows it (a Q8_0 or Q4_0 down), gate/up
+        // runs on k_gemm_f16 writing fp32 act and the down projection on the fp32 GEMM,
         // over the same 64-token tiles.
         const PrefillPlan plan = prefill_plan(L, T);
         const bool f16gu = plan.f16gu, f16 = plan.f16, merge = plan.merge, gu8 = plan.gu8, dn8 = plan.dn8;

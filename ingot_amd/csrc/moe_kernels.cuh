@@ -2743,8 +2743,8 @@ struct BStream {
     }
 };
 
-// Grouped GEMM on f16 MFMA for Q4_K, IQ3_XXS and IQ4_NL weights (see the
-// block comment above). e_shared names the tile expert id whose weights are
+// Grouped GEMM on f16 MFMA for weights of the formats of BStream (Q8_0, the k-quants
+// Q4_K, Q5_K and Q6_K, and the IQ formats; see the block comment above). e_shared names the tile expert id whose weights are
 // ws0/ws1 (the shared expert, run in the same launch); no tile carries it when
 // it is 0xffffffff. AORD (gate/up only) is the column order in which act is
 // stored: the order the down projection's format reads (a_pos).
