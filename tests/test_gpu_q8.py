@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from ingot_amd import configs as CF
-from ingot_amd.moe import IQ2_XS, IQ4_NL, Q4_K, Q6_K, Q8_0, STAGE_DOWN, STAGE_GATEUP, LayerSpec, Matrix, MoeLayer
+from ingot_amd.moe import IQ2_XS, IQ4_NL, Q4_K, Q6_K, Q8_0, STAGE_DOWN, STAGE_GATEUP, Gpu, LayerSpec, Matrix, MoeLayer
 from test_gpu_small_tiles import LOADS, assert_rows_close, routed_inputs
 from util import check_layer
 
@@ -92,11 +92,12 @@ def test_q8_expert_of_4_gib(gpu):
     layer.destroy()
 
 
-def test_q8_copies_leave_room(gpu):
+def test_q8_copies_leave_room():
     """The second copies of a Q8_0 layer's weights are not made on a nearly full card (a
     sixteenth of it is left), and the layer computes the same without them."""
     spec = CF.make_layer(67, 0, 1024, 32, 4, 512, Q8_0, Q8_0)
     x = CF.inputs(67, 70, 1024)
+    gpu = Gpu(0)  # its own: a failed allocation closes a context
     full, roomy = MoeLayer(gpu, spec), MoeLayer(gpu, spec)
     bytes_ = full.weight_bytes()
     roomy.reserve(70)
@@ -118,6 +119,7 @@ def test_q8_copies_leave_room(gpu):
     assert np.array_equal(out, roomy(x)[0]) and roomy.weight_bytes() > 2 * bytes_ - (1 << 20)
     for layer in (full, roomy, clone):
         layer.destroy()
+    gpu.close()
 
 
 @pytest.mark.parametrize("scale", [1e-12, 1e-4, 1e4, 1e12])

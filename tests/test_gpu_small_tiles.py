@@ -67,6 +67,15 @@ def test_tile_loads(gpu, oracle, gk, dk, F, shared):
         cached.destroy()
 
 
+def wide_spec(gk, dk, shared):
+    """64 experts of 1792, four of them distinct."""
+    spec = CF.make_layer(66, 0, 1024, 4, 1, 1792, gk, dk, shared_ffn=1792 if shared else 0)
+    spec.experts = 64
+    for m in ("gate", "up", "down"):
+        setattr(spec, m, getattr(spec, m).select([(5 * e) % 4 for e in range(64)]))
+    return spec
+
+
 # 64 experts of 1792 (28 gate/up blocks a tile): the dispatch chooses from 686 pairs on, k_gemm_f16 above
 # 54 tiles of 16 pairs if they are more than 7 to 4 64-pair tiles.
 @pytest.mark.parametrize("loads,shared,f16", [
@@ -76,11 +85,8 @@ def test_tile_loads(gpu, oracle, gk, dk, F, shared):
     ([250, 250, 240] + [1] * 27, True, True)])
 @pytest.mark.parametrize("gk,dk", [(Q4_K, Q6_K), (Q8_0, Q8_0)])
 def test_dispatch_chooses_by_tiles(gpu, oracle, gk, dk, loads, shared, f16):
-    H, E, F = 1024, 64, 1792
-    spec = CF.make_layer(66, 0, H, 4, 1, F, gk, dk, shared_ffn=F if shared else 0)
-    spec.experts = E
-    for m in ("gate", "up", "down"):
-        setattr(spec, m, getattr(spec, m).select([(5 * e) % 4 for e in range(E)]))
+    spec = wide_spec(gk, dk, shared)
+    H, E = spec.hidden, spec.experts
     loads = loads + [0] * (E - len(loads))
     x = routed_inputs(spec, loads, H, 66)
     res, cached = MoeLayer(gpu, spec), MoeLayer(gpu, spec, cache_slots=40)
@@ -92,3 +98,30 @@ def test_dispatch_chooses_by_tiles(gpu, oracle, gk, dk, loads, shared, f16):
     assert np.array_equal(out, cached(x)[0])
     res.destroy()
     cached.destroy()
+
+
+def test_captured_forward_chooses_at_each_replay(gpu):
+    """One graph, replayed with inputs for which the dispatch chooses either kernel."""
+    spec = wide_spec(Q4_K, Q6_K, True)
+    T, H, E = 768, spec.hidden, spec.experts
+    xs = [routed_inputs(spec, loads + [0] * (E - len(loads)), H, 67)
+          for loads in ([12] * 64, [250, 250, 241] + [1] * 27, [256, 256, 256])]
+    eager, layer = MoeLayer(gpu, spec), MoeLayer(gpu, spec)
+    refs = [eager(x)[0] for x in xs]
+    layer.reserve(T)
+    dx, dout = gpu.buffer(4 * T * H), gpu.buffer(4 * T * H)
+    gpu.graph_begin()
+    layer.forward(dx, T, dout)
+    graph = gpu.graph_end()
+    for i in (0, 1, 0, 2, 1):
+        dx.upload(xs[i])
+        graph.launch()
+        gpu.synchronize()
+        assert np.array_equal(dout.download(np.float32, T * H).reshape(T, H), refs[i])
+        gemm = ("k_gemm_small", "k_gemm_f16", "k_gemm_f16")[i]  # 112 tiles to 76; 123 to 51; 96 to 24
+        assert layer.stage_kernel(STAGE_GATEUP) == f"{gemm}<gate_up>"
+        assert np.array_equal(eager(xs[i])[0], refs[i])
+    gpu.check_device_flags()
+    graph.destroy()
+    eager.destroy()
+    layer.destroy()
